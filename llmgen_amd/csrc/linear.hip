@@ -1,0 +1,353 @@
+// linear.hip -- y [M, N] = x [M, K] * w [N, K]^T in the reference CPU backend's order (hip_linear).
+//
+// The reference (src/backend/cpu/linear.zig:7-28) forms every output as one f32 sum over k = 0 .. K-1, a rounded
+// multiply and a rounded add per term.  The product of two bf16 values has at most 16 significant bits, so f32 holds
+// it exactly unless it leaves the exponent range; then multiply-and-add is a fused multiply-add, and
+// v_mfma_f32_16x16x4_f32 is exactly that: four fused multiply-adds per output, k ascending, each rounded to nearest
+// even, denormals kept (the bf16 matrix instructions are not: they add several products before they round).  The
+// K sum cannot be split and its order cannot change, so the work is spread over outputs only.
+//
+// Exactness is checked, not assumed: each staged value must be zero or lie in a window of 128 exponents
+// (x: [2^-63, 2^65), w: [2^-67, 2^61)), so that a product is below 2^126 and a multiple of 2^-144.  The check is an
+// add and an AND per pair of values (adding 64 or 68 to the exponent field sets its top bit exactly inside the
+// window); zeros fail it and are sorted out in a second look at the rows that were staged.  A tile that holds any
+// other value (infinities and NaN among them) is computed again with separate multiplies and adds.
+//
+// What bounds it.  f32 matrix instructions run at 155 TFLOP/s (1/16 of bf16) and share their issue slots with the
+// VALU: measured, every VALU instruction beside them adds its full 4 cycles.  So operands are widened to f32 once per
+// tile on their way into LDS (bf16 rows -> registers -> f32 rows in LDS, laid out so that one ds_read_b128 gives a
+// lane its operand of four instructions) and the product loop holds nothing but LDS reads and matrix instructions.
+// Loads run PF chunks ahead of the staging, staging two chunks ahead of the products and the LDS reads one chunk
+// ahead, so that one barrier per chunk is all a wave waits for.
+//
+// Small steps (decode) are bound by the chain of one output instead: 8 cycles per k, 3.4 us at K = 1024.  There a
+// wave owns a single 16 x 16 tile and staging is left to producer waves of the same workgroup, which sit on the other
+// SIMDs, so the chain's SIMD does nothing else (K = 3072, N = 1024, 32 rows: 17 us; with the staging in the same wave
+// 27 us; before, one output per lane with 256-column workgroups: 400 us).
+#include "hip_common.h"
+
+#include <type_traits>
+
+#pragma clang fp contract(off)
+
+namespace {
+
+// Added to a pair of bf16 values, sets bit 14 of each half exactly where the exponent field lies in the window.
+constexpr uint32_t LIN_X_BIAS = 0x20002000u;  // exponent field 64..191: [2^-63, 2^65)
+constexpr uint32_t LIN_W_BIAS = 0x22002200u;  // exponent field 60..187: [2^-67, 2^61)
+constexpr uint32_t LIN_IN = 0x40004000u;
+
+// One value: zero, or inside the window of its operand.
+__device__ __forceinline__ bool lin_half_ok(uint32_t h, uint32_t bias) {
+    return (h & 0x7fffu) == 0 || (((h & 0x7fffu) + (bias & 0x7fffu)) & 0xC000u) == 0x4000u;
+}
+
+struct LinArgs {
+    void *y;
+    const bf16_t *x, *w;
+    int M, N, K, y_f32, vec_out, tiles_m, tiles_n;
+};
+
+// A workgroup's tile: WM x WN waves of MT x NT blocks of 16 x 16 outputs, PW extra waves that only stage (0: every
+// wave stages), KC values of k per LDS chunk.
+template <int MT, int NT, int WM, int WN, int PW, int KC>
+struct LinTile {
+    static constexpr int TM = WM * MT * 16, TN = WN * NT * 16, ROWS = TM + TN;
+    static constexpr int WAVES = WM * WN, THREADS = (WAVES + PW) * 64, STAGERS = (PW ? PW : WAVES) * 64;
+    static constexpr int UNITS = KC / 16;  // 16 consecutive k of a row: one staging slot
+    static constexpr int WORK = ROWS * UNITS, SLOTS = (WORK + STAGERS - 1) / STAGERS;
+    static constexpr int STRIDE = KC + 4;  // f32 per staged row
+    static constexpr int LDS = 2 * ROWS * STRIDE * 4;
+    // whether slot s of a staging thread has work (whole waves drop out of the last slot)
+    static __device__ __forceinline__ bool has(int id, int s) {
+        return (s + 1) * STAGERS <= WORK || id + s * STAGERS < WORK;
+    }
+};
+
+template <int MT, int NT, int WM, int WN, int PW, int KC, int PF>
+__global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinArgs a) {
+    using T = LinTile<MT, NT, WM, WN, PW, KC>;
+    static_assert(PF % 2 == 0, "chunk parity names the LDS buffer");
+    __shared__ __attribute__((aligned(16))) float lds[2][T::ROWS * T::STRIDE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // tiles in order of columns, each XCD (block index mod 8) a contiguous range of them
+    const int tiles = a.tiles_m * a.tiles_n;
+    const int per = tiles >> 3, rem = tiles & 7, xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+    const int tile = xcd * per + min(xcd, rem) + at;
+    const int n0 = tile / a.tiles_m * T::TN, m0 = tile % a.tiles_m * T::TM;
+    const int K = a.K, full = K / KC, tail = K - full * KC;
+
+    // ---- staging: raw bf16 rows -> f32 in LDS, each 16 k of a row as [k % 4][k / 4]
+    const int sid = PW ? tid - T::WAVES * 64 : tid;
+    const bf16_t *src[T::SLOTS];
+    int dst[T::SLOTS], koff[T::SLOTS];
+    bool is_w[T::SLOTS];
+    u32x4_t raw[PF][T::SLOTS][2];
+    int ahead = 0;  // next chunk to load
+    uint32_t bad = 0;
+    auto load = [&](u32x4_t (&r)[T::SLOTS][2]) {
+#pragma unroll
+        for (int s = 0; s < T::SLOTS; ++s)
+            if (T::has(sid, s))
+#pragma unroll
+                for (int h = 0; h < 2; ++h) r[s][h] = ld16(src[s] + h * 8);
+        const int step = ++ahead < full ? KC : 0;  // past the last full chunk: that chunk again
+#pragma unroll
+        for (int s = 0; s < T::SLOTS; ++s) src[s] += step;
+    };
+    // the last K % KC values of each row, zeros beyond them; the pointers stand at the last full chunk (or at k 0)
+    auto load_tail = [&](u32x4_t (&r)[T::SLOTS][2]) {
+        const int base = full > 0 ? KC : 0;
+#pragma unroll
+        for (int s = 0; s < T::SLOTS; ++s)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                r[s][h] = u32x4_t{0u, 0u, 0u, 0u};
+                if (T::has(sid, s) && koff[s] + h * 8 < tail) r[s][h] = ld16(src[s] + base + h * 8);
+            }
+    };
+    auto stage = [&](const u32x4_t (&r)[T::SLOTS][2], int buf) {
+        uint32_t in = LIN_IN;
+#pragma unroll
+        for (int s = 0; s < T::SLOTS; ++s) {
+            if (!T::has(sid, s)) continue;
+            const uint32_t bias = is_w[s] ? LIN_W_BIAS : LIN_X_BIAS;
+            float f[16];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) in &= r[s][h][i] + bias;
+                unpack_bf16x8(r[s][h], f + 8 * h);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<f32x4_t *>(&lds[buf][dst[s] + q * 4]) = f32x4_t{f[q], f[4 + q], f[8 + q], f[12 + q]};
+        }
+        if (__builtin_expect(__ballot(in != LIN_IN) != 0, 0)) {
+#pragma unroll
+            for (int s = 0; s < T::SLOTS; ++s) {
+                if (!T::has(sid, s)) continue;
+                const uint32_t bias = is_w[s] ? LIN_W_BIAS : LIN_X_BIAS;
+                for (int h = 0; h < 2; ++h)
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t d = r[s][h][i];
+                        bad |= !(lin_half_ok(d & 0xffffu, bias) && lin_half_ok(d >> 16, bias));
+                    }
+            }
+        }
+    };
+
+    // ---- products
+    const int wm = wave % WM, wn = wave / WM;
+    const int frag = (lane & 15) * T::STRIDE + (lane >> 4) * 4;
+    const int wbase = wn * NT * 16 * T::STRIDE + frag, xbase = (T::TN + wm * MT * 16) * T::STRIDE + frag;
+    f32x4_t acc[MT][NT];
+    f32x4_t wf[2][T::UNITS][NT], xf[2][T::UNITS][MT];
+    auto fetch = [&](int set) {
+        const float *b = lds[set];
+#pragma unroll
+        for (int s = 0; s < T::UNITS; ++s) {
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                wf[set][s][n] = *reinterpret_cast<const f32x4_t *>(b + wbase + n * 16 * T::STRIDE + s * 16);
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+                xf[set][s][m] = *reinterpret_cast<const f32x4_t *>(b + xbase + m * 16 * T::STRIDE + s * 16);
+        }
+    };
+    auto compute = [&](int set) {
+#pragma unroll
+        for (int s = 0; s < T::UNITS; ++s)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n)
+                        acc[m][n] =
+                            __builtin_amdgcn_mfma_f32_16x16x4f32(wf[set][s][n][j], xf[set][s][m][j], acc[m][n], 0, 0, 0);
+    };
+
+    // Step i: the products of chunk i, the fragments of chunk i + 1, the staging of chunk i + 2, the loads of chunk
+    // i + 2 + PF.
+    auto run = [&](auto stager, auto multiplier) {
+        constexpr bool S = decltype(stager)::value, C = decltype(multiplier)::value;
+        const int chunks = full + (tail > 0);
+        if constexpr (S) {
+#pragma unroll
+            for (int s = 0; s < T::SLOTS; ++s) {
+                const int i = sid + s * T::STAGERS, row = min(i / T::UNITS, T::ROWS - 1), u = i % T::UNITS;
+                is_w[s] = row < T::TN;
+                const long r = is_w[s] ? min(n0 + row, a.N - 1) : min(m0 + row - T::TN, a.M - 1);
+                koff[s] = u * 16;
+                src[s] = (is_w[s] ? a.w : a.x) + r * K + u * 16;
+                dst[s] = row * T::STRIDE + u * 16;
+            }
+            if (full > 0) {
+#pragma unroll
+                for (int p = 0; p < PF; ++p) load(raw[p]);
+            }
+            if (full == 0) load_tail(raw[0]);
+            stage(raw[0], 0);
+            if (full > 0) load(raw[0]);
+        }
+        if constexpr (C) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int n = 0; n < NT; ++n) acc[m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+        __syncthreads();
+        if constexpr (C) fetch(0);
+        if constexpr (S) {
+            if (full == 1 && tail) load_tail(raw[1]);
+            if (chunks > 1) stage(raw[1], 1);
+            if (full > 0) load(raw[1]);
+        }
+        __syncthreads();
+        int i = 0;
+        for (; i + PF + 2 <= full; i += PF) {
+#pragma unroll
+            for (int p = 0; p < PF; ++p) {
+                if constexpr (C) fetch((p + 1) & 1);
+                if constexpr (S) {
+                    stage(raw[(p + 2) % PF], p & 1);
+                    load(raw[(p + 2) % PF]);
+                }
+                if constexpr (C) compute(p & 1);
+                __syncthreads();
+            }
+        }
+        // at most PF + 2 chunks are left, the last of them perhaps partial
+        if constexpr (S) {
+#pragma unroll
+            for (int r = 2; r < PF + 2; ++r)
+                if (tail && i + r == full) load_tail(raw[r % PF]);
+        }
+#pragma unroll
+        for (int p = 0; p < PF + 2; ++p)
+            if (i + p < chunks) {
+                if constexpr (C)
+                    if (i + p + 1 < chunks) fetch((p + 1) & 1);
+                if constexpr (S)
+                    if (i + p + 2 < chunks) stage(raw[(p + 2) % PF], p & 1);
+                if constexpr (C) compute(p & 1);
+                __syncthreads();
+            }
+    };
+    if constexpr (PW == 0) {
+        run(std::true_type{}, std::true_type{});
+    } else {
+        if (__builtin_amdgcn_readfirstlane(wave) < T::WAVES)
+            run(std::false_type{}, std::true_type{});
+        else
+            run(std::true_type{}, std::false_type{});
+    }
+    // D of the instruction: columns are rows of x, a lane's four values are consecutive columns of y
+    auto put = [&](int m, int n, float v) {
+        const long o = (long)m * a.N + n;
+        if (a.y_f32)
+            static_cast<float *>(a.y)[o] = v;
+        else
+            static_cast<bf16_t *>(a.y)[o] = __builtin_bit_cast(bf16_t, (__bf16)v);
+    };
+    if (__builtin_expect(__syncthreads_or((int)bad), 0)) {
+        // a value outside its window: the reference's separate multiplies and adds
+        for (int i = tid; i < T::TM * T::TN; i += T::THREADS) {
+            const int m = m0 + i / T::TN, n = n0 + i % T::TN;
+            if (m >= a.M || n >= a.N) continue;
+            const bf16_t *xr = a.x + (long)m * K, *wr = a.w + (long)n * K;
+            float s = 0.0f;
+            for (int k = 0; k < K; k += 8) {
+                float xv[8], wv[8];
+                unpack_bf16x8(ld16(xr + k), xv);
+                unpack_bf16x8(ld16(wr + k), wv);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) s = s + xv[e] * wv[e];
+            }
+            put(m, n, s);
+        }
+        return;
+    }
+    if (PW && wave >= T::WAVES) return;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int row = m0 + (wm * MT + m) * 16 + (lane & 15);
+        if (row >= a.M) continue;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const int col = n0 + (wn * NT + n) * 16 + (lane >> 4) * 4;
+            if (a.vec_out && col < a.N) {
+                const long o = (long)row * a.N + col;
+                if (a.y_f32)
+                    *reinterpret_cast<f32x4_t *>(static_cast<float *>(a.y) + o) = acc[m][n];
+                else
+                    *reinterpret_cast<u32x2_t *>(static_cast<bf16_t *>(a.y) + o) =
+                        u32x2_t{pack_bf16x2(acc[m][n][0], acc[m][n][1]), pack_bf16x2(acc[m][n][2], acc[m][n][3])};
+            } else {
+                for (int r = 0; r < 4; ++r)
+                    if (col + r < a.N) put(row, col + r, acc[m][n][r]);
+            }
+        }
+    }
+}
+
+template <int MT, int NT, int WM, int WN, int PW, int KC, int PF>
+void linear_launch(LinArgs a) {
+    using T = LinTile<MT, NT, WM, WN, PW, KC>;
+    a.tiles_m = (a.M + T::TM - 1) / T::TM;
+    a.tiles_n = (a.N + T::TN - 1) / T::TN;
+    linear_kernel<MT, NT, WM, WN, PW, KC, PF><<<a.tiles_m * a.tiles_n, T::THREADS, 0, g_llmgen_stream>>>(a);
+}
+
+// Tiles of the throughput-bound sizes.  A launch takes about as long as the CU with the most tiles:
+// ceil(tiles / CUs) * blocks of a tile / rate, where `rate` is the share of the matrix cores' peak that the tile
+// reached on sizes it fits (launch time taken off): 0.64 for 32 x 32 (M = 2051, N = K = 1024: 50.8 us), 0.75 for
+// 64 x 64 (997 x 3072 x 1024: 58.2 us), 0.76 for 64 x 192 and 96 x 192 (57.4 us; 2051 x 2048 x 1024: 83.8 us) and
+// 0.81 for 128 x 128 (2048 x 6144 x 2048: 407 us = 127 TFLOP/s).  Larger tiles stage less per product but quantise
+// coarser; the best of the five by this rule was within 4 % of the best of 33 measured tiles on 12 sizes from
+// 200 x 3072 x 1024 to 3000 x 4096 x 2560.
+struct LinChoice {
+    int tm, tn;
+    float rate;
+    void (*launch)(LinArgs);
+};
+const LinChoice LIN_CHOICES[] = {{32, 32, 0.64f, linear_launch<1, 1, 2, 2, 0, 64, 2>},
+                                 {64, 64, 0.75f, linear_launch<2, 2, 2, 2, 0, 32, 2>},
+                                 {64, 192, 0.76f, linear_launch<2, 3, 2, 4, 0, 32, 2>},
+                                 {96, 192, 0.765f, linear_launch<3, 3, 2, 4, 0, 32, 2>},
+                                 {128, 128, 0.81f, linear_launch<4, 2, 2, 4, 0, 32, 2>}};
+
+void linear_dispatch(const LinArgs &a) {
+    const long blocks = (long)((a.M + 15) / 16) * ((a.N + 15) / 16);
+    const int cus = llmgen_num_cus();
+    // At most one 16 x 16 block per CU: one block and three staging waves a workgroup (8.2 us at 1 x 1024 x 1024,
+    // 17.7 us at 32 x 1024 x 3072; two blocks and two staging waves 9.8 and 24 us).  At most two: two blocks and two
+    // staging waves (11.3 us at 32 x 3072 x 1024; single blocks 12.6 us).
+    if (blocks <= cus) return linear_launch<1, 1, 1, 1, 3, 128, 2>(a);
+    if (blocks <= 2 * cus) return linear_launch<1, 1, 1, 2, 2, 64, 4>(a);
+    // Up to 16 rows and many columns: bound by the read of w; small workgroups, eight of them a CU (8 x 151936 x
+    // 1024: 78 us; 32 x 32 tiles, half of them empty, 108 us).
+    if (a.M <= 16) return linear_launch<1, 1, 1, 2, 0, 64, 2>(a);
+    const LinChoice *best = nullptr;
+    float cost = 0.f;
+    for (const LinChoice &c : LIN_CHOICES) {
+        const long tiles = (long)((a.M + c.tm - 1) / c.tm) * ((a.N + c.tn - 1) / c.tn);
+        const float t = (float)((tiles + cus - 1) / cus) * (float)(c.tm * c.tn) / c.rate;
+        if (!best || t < cost) best = &c, cost = t;
+    }
+    best->launch(a);
+}
+
+}  // namespace
+
+extern "C" void hip_linear(void *y, int y_f32, const uint16_t *x, const uint16_t *w, int M, int N, int K) {
+    if (M <= 0 || N <= 0) return;
+    if (K <= 0 || K % 8 != 0) {
+        fprintf(stderr, "llmgen: hip_linear: K must be a positive multiple of 8\n");
+        return;
+    }
+    // four outputs of a row are stored as one word where each such group is aligned for it
+    const int vec = N % 4 == 0 && (uintptr_t)y % (y_f32 ? 16 : 8) == 0;
+    linear_dispatch(LinArgs{y, x, w, M, N, K, y_f32, vec, 0, 0});
+}

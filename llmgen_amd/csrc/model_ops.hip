@@ -1,4 +1,4 @@
-// model_ops.hip -- the non-attention ops of the Qwen3 forward (embedding, RMSNorm, linear, NEOX RoPE, SiLU,
+// model_ops.hip -- the non-attention ops of the Qwen3 forward except linear (embedding, RMSNorm, NEOX RoPE, SiLU,
 // add, mul, gather_last, sampling) for the end-to-end greedy-token check, and the fused q/k norm + RoPE + KV
 // write that replaces five of them before attention.
 //
@@ -55,66 +55,6 @@ __global__ void __launch_bounds__(64) rmsnorm_kernel(bf16_t *out, const bf16_t *
     for (int h = threadIdx.x; h < D; h += 64) {
         const float normed = bf2f(f2bf(row[h] * scale));
         out[r * D + h] = f2bf(normed * w[h]);
-    }
-}
-
-// ---------------------------------------------------------------------------------------------- linear
-// y[m][n] = sum_k x[m][k] * w[n][k], k ascending.  A workgroup owns 256 output columns (one per thread) and
-// LIN_MB rows; K advances in tiles of LIN_KT: the W tile (256 x LIN_KT bf16) and the x tile (LIN_MB x LIN_KT,
-// as f32) are staged in LDS with coalesced 16-byte loads.  W rows are padded to an odd number of dwords so the
-// 64 lanes of a wave read 64 different banks.  Each thread keeps LIN_MB independent chains.
-constexpr int LIN_N = 256, LIN_MB = 8, LIN_KT = 32;
-constexpr int LIN_WSTRIDE = LIN_KT / 2 + 1;  // dwords per padded W row (17)
-
-__global__ void __launch_bounds__(LIN_N) linear_kernel(void *y, int y_f32, const bf16_t *x, const bf16_t *w, int M,
-                                                       int N, int K) {
-    __shared__ uint32_t ws[LIN_N * LIN_WSTRIDE];
-    __shared__ float xs[LIN_MB][LIN_KT];
-    const int tid = threadIdx.x;
-    const int n0 = blockIdx.x * LIN_N, m0 = blockIdx.y * LIN_MB;
-    const int n = n0 + tid;
-    const int mrows = min(LIN_MB, M - m0);
-    float acc[LIN_MB];
-#pragma unroll
-    for (int m = 0; m < LIN_MB; ++m) acc[m] = 0.0f;
-
-    for (int k0 = 0; k0 < K; k0 += LIN_KT) {
-        const int kt = min(LIN_KT, K - k0);  // multiple of 8
-        // W tile: 256 rows x (kt / 8) chunks of 16 bytes
-        for (int i = tid; i < LIN_N * (LIN_KT / 8); i += LIN_N) {
-            const int r = i / (LIN_KT / 8), c = i % (LIN_KT / 8);
-            u32x4_t v = {0u, 0u, 0u, 0u};
-            if (n0 + r < N && c * 8 < kt) v = ld16(w + (long)(n0 + r) * K + k0 + c * 8);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) ws[r * LIN_WSTRIDE + c * 4 + j] = v[j];
-        }
-        // x tile: mrows x (kt / 8) chunks
-        for (int i = tid; i < LIN_MB * (LIN_KT / 8); i += LIN_N) {
-            const int r = i / (LIN_KT / 8), c = i % (LIN_KT / 8);
-            float f[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-            if (r < mrows && c * 8 < kt) unpack_bf16x8(ld16(x + (long)(m0 + r) * K + k0 + c * 8), f);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) xs[r][c * 8 + j] = f[j];
-        }
-        __syncthreads();
-        for (int kk = 0; kk < kt; kk += 2) {
-            const uint32_t wp = ws[tid * LIN_WSTRIDE + (kk >> 1)];
-            const float w0 = bf16lo_to_f32(wp), w1 = bf16hi_to_f32(wp);
-#pragma unroll
-            for (int m = 0; m < LIN_MB; ++m) {
-                acc[m] = acc[m] + xs[m][kk] * w0;
-                acc[m] = acc[m] + xs[m][kk + 1] * w1;
-            }
-        }
-        __syncthreads();
-    }
-    if (n >= N) return;
-    for (int m = 0; m < mrows; ++m) {
-        const long o = (long)(m0 + m) * N + n;
-        if (y_f32)
-            static_cast<float *>(y)[o] = acc[m];
-        else
-            static_cast<bf16_t *>(y)[o] = f2bf(acc[m]);
     }
 }
 
@@ -274,16 +214,6 @@ void hip_rmsnorm(uint16_t *out, const uint16_t *x, const float *w, long rows, in
         return;
     }
     rmsnorm_kernel<<<(unsigned)rows, 64, 0, g_llmgen_stream>>>(out, x, w, D, eps);
-}
-
-void hip_linear(void *y, int y_f32, const uint16_t *x, const uint16_t *w, int M, int N, int K) {
-    if (M <= 0 || N <= 0) return;
-    if (K <= 0 || K % 8 != 0) {
-        reject("hip_linear: K must be a positive multiple of 8");
-        return;
-    }
-    const dim3 grid((N + LIN_N - 1) / LIN_N, (M + LIN_MB - 1) / LIN_MB);
-    linear_kernel<<<grid, LIN_N, 0, g_llmgen_stream>>>(y, y_f32, x, w, M, N, K);
 }
 
 void hip_rope(uint16_t *out, const uint16_t *x, const float *cos_tab, const float *sin_tab, const int32_t *positions,

@@ -1,0 +1,83 @@
+"""hip_linear against the oracle, bit for bit, on every tile shape of its dispatch (llmgen_amd/csrc/linear.hip): edges of
+the tiles, K remainders, unaligned outputs, and values outside the windows in which products are exact."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from llmgen_amd._lib import lib
+
+pytestmark = pytest.mark.gpu
+
+
+def run(x, w, y_f32, offset=0):
+    """hip_linear on bf16 bits; ``offset`` shifts the output by that many values from its aligned start."""
+    M, N, K = x.shape[0], w.shape[0], x.shape[1]
+    xd, wd = (torch.from_numpy(a.view(np.int16)).cuda() for a in (x, w))
+    out = torch.full((M * N + offset + 8,), 77, dtype=torch.float32 if y_f32 else torch.int16, device="cuda")
+    lib().hip_linear(out.data_ptr() + offset * out.element_size(), int(y_f32), xd.data_ptr(), wd.data_ptr(), M, N, K)
+    torch.cuda.synchronize()
+    assert lib().hip_last_error() == 0
+    got = out.cpu().numpy()
+    assert (got[:offset] == 77).all() and (got[offset + M * N:] == 77).all(), "wrote outside y"
+    got = got[offset:offset + M * N].reshape(M, N)
+    return got if y_f32 else got.view(np.uint16)
+
+
+def check(x, w, y_f32, offset=0):
+    got, ref = run(x, w, y_f32, offset), O.linear(x, w, out_bf16=not y_f32)
+    if y_f32:
+        nan = np.isnan(ref)
+        got, ref, isnan = got.view(np.uint32), ref.view(np.uint32), np.isnan(got)
+    else:
+        nan, isnan = ((a & 0x7FFF) > 0x7F80 for a in (ref, got))
+    np.testing.assert_array_equal(isnan, nan)
+    np.testing.assert_array_equal(got[~nan], ref[~nan])
+
+
+def draw(rng, *shape, std=1.0):
+    return O.f32_to_bf16((std * rng.standard_normal(shape)).astype(np.float32))
+
+
+# (M, N, K): one 16 x 16 block a workgroup, two blocks, up to 16 rows of many columns, then 32 x 32, 64 x 64, 64 x 192,
+# 96 x 192 and 128 x 128 tiles
+@pytest.mark.parametrize("M,N,K", [(1, 1, 8), (1, 16, 128), (17, 100, 24), (16, 1024, 1000), (3, 2049, 264),
+                                   (33, 1700, 72), (40, 2000, 320), (16, 8200, 40), (5, 9001, 200), (50, 3000, 200),
+                                   (129, 1031, 64), (512, 2048, 72), (1000, 3060, 40), (2051, 2048, 24),
+                                   (2048, 6144, 16)])
+def test_linear_tiles_bit_exact(gpu, M, N, K):
+    rng = np.random.default_rng(M + 3 * N + K)
+    check(draw(rng, M, K), draw(rng, N, K, std=0.05), y_f32=M % 2 == 1)
+
+
+@pytest.mark.parametrize("N,offset", [(64, 0), (64, 1), (64, 2), (62, 0), (63, 3)])
+@pytest.mark.parametrize("y_f32", [False, True])
+def test_linear_any_output_alignment(gpu, N, offset, y_f32):
+    rng = np.random.default_rng(N + offset)
+    check(draw(rng, 19, 48), draw(rng, N, 48), y_f32, offset)
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 70, 136), (40, 2000, 72), (12, 8300, 72), (200, 1100, 200), (512, 2048, 40)])
+@pytest.mark.parametrize("what", ["zeros", "tiny", "huge", "nonfinite", "edges"])
+def test_linear_values_outside_the_exact_window(gpu, M, N, K, what):
+    """Zeros stay on the fast path; values whose products leave f32's exact range (or are not finite) must take the
+    separate multiply and add.  Only some tiles hold such values, so both paths run in one launch."""
+    rng = np.random.default_rng(M * 5 + len(what))
+    x, w = draw(rng, M, K), draw(rng, N, K, std=0.1)
+    special = {"zeros": [0x0000, 0x8000], "tiny": [0x0001, 0x8001, 0x0080, 0x1000, 0x9A00],
+               "huge": [0x7F00, 0xFF7F, 0x7E80, 0xF000], "nonfinite": [0x7F80, 0xFF80, 0x7FC0],
+               # the first and last exponents inside and outside the windows of x (64..191) and w (60..187)
+               "edges": [e << 7 for e in (59, 60, 63, 64, 187, 188, 191, 192)]}[what]
+    for a in (x, w):
+        n = max(1, a.size // 50) if what == "zeros" else 6
+        at = rng.integers(0, a.size, n)
+        a.reshape(-1)[at] = rng.choice(np.array(special, np.uint16), n)
+    if what == "zeros":
+        x[0], w[-1] = 0, 0
+    if what in ("tiny", "edges"):  # whole rows of them, so that the sums are tiny too
+        x[M // 2] = rng.choice(np.array(special, np.uint16), K)
+        w[N // 2] = rng.choice(np.array(special, np.uint16), K)
+    check(x, w, y_f32=True)
+    check(x, w, y_f32=False)
