@@ -1,0 +1,90 @@
+"""The row and element ops of llmgen_amd/csrc/model_ops.hip at the edges of their launch rules, bit for bit against the
+oracle: rows per wave of RMSNorm, vector and scalar parts of the elementwise ops, slices of a sampled row."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from llmgen_amd._lib import lib
+
+pytestmark = pytest.mark.gpu
+
+
+def up(a):
+    a = np.ascontiguousarray(a)
+    return torch.from_numpy(a.view(np.int16) if a.dtype == np.uint16 else a).cuda()
+
+
+def down(t):
+    torch.cuda.synchronize()
+    assert lib().hip_last_error() == 0
+    return t.cpu().numpy().view(np.uint16)
+
+
+def draw(rng, *shape, std=1.0):
+    return O.f32_to_bf16((std * rng.standard_normal(shape)).astype(np.float32))
+
+
+# one, two, four and eight rows a wave, the last wave partly empty; D below, at and off the chain's step of 64
+@pytest.mark.parametrize("rows,D", [(1, 8), (3, 72), (5, 8192), (2049, 136), (2051, 4096), (4099, 1000), (4097, 1024),
+                                    (8195, 128), (8193, 512), (8193, 520)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_rmsnorm_rows_per_wave(gpu, rows, D, offset):
+    rng = np.random.default_rng(rows + D)
+    x, g = draw(rng, rows, D, std=2.0), (1 + 0.1 * rng.standard_normal(D)).astype(np.float32)
+    out = torch.zeros(rows * D + offset + 8, dtype=torch.int16, device="cuda")
+    xd, gd = up(x), up(g)
+    lib().hip_rmsnorm(out.data_ptr() + 2 * offset, xd.data_ptr(), gd.data_ptr(), rows, D, 1e-6)
+    got = down(out)
+    np.testing.assert_array_equal(got[offset:offset + rows * D].reshape(rows, D), O.rmsnorm(x, g, 1e-6))
+    assert not got[:offset].any() and not got[offset + rows * D:].any()
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 2047, 2048, 2049, 4101])
+@pytest.mark.parametrize("offset", [0, 1, 4])
+def test_elementwise_tails_and_alignment(gpu, n, offset):
+    rng = np.random.default_rng(n)
+    a, b = draw(rng, n, std=4.0), draw(rng, n, std=2.0)
+    ad, bd = (torch.cat([torch.zeros(offset, dtype=torch.int16, device="cuda"), up(t)]) for t in (a, b))
+    for name, ref in (("add", O.add(a, b)), ("mul", O.mul(a, b))):
+        out = torch.zeros(n + 16, dtype=torch.int16, device="cuda")
+        getattr(lib(), "hip_" + name)(out.data_ptr(), ad.data_ptr() + 2 * offset, bd.data_ptr() + 2 * offset, n)
+        got = down(out)
+        np.testing.assert_array_equal(got[:n], ref)
+        assert not got[n:].any()
+
+
+def test_silu_every_value(gpu):
+    """All 65536 inputs against x / (1 + exp(-x)) with exp rounded once to f32, as a correctly rounded expf gives it."""
+    bits = np.arange(65536, dtype=np.uint32).astype(np.uint16)
+    out = torch.zeros(65536, dtype=torch.int16, device="cuda")
+    lib().hip_silu(out.data_ptr(), up(bits).data_ptr(), 65536)
+    got, v = down(out), O.bf16_to_f32(bits)
+    with np.errstate(all="ignore"):
+        e = np.exp(-v.astype(np.float64)).astype(np.float32)
+        ref = O.f32_to_bf16(v / (np.float32(1) + e))
+    nan = (ref & 0x7FFF) > 0x7F80
+    np.testing.assert_array_equal((got & 0x7FFF) > 0x7F80, nan)
+    np.testing.assert_array_equal(got[~nan], ref[~nan])
+
+
+# one slice, several; rows that start unaligned (odd V); rows shorter than a vector
+@pytest.mark.parametrize("S,V", [(1, 1), (3, 7), (2, 8191), (5, 16384), (3, 16391), (4, 65549), (1, 300007)])
+def test_sample_slices(gpu, S, V):
+    rng = np.random.default_rng(S + V)
+    lg = draw(rng, S, V)
+    lg[0, [V // 3, V - 1]] = O.f32_to_bf16(np.array([9.0], np.float32))[0]  # a tie, the second in the last slice
+    if S > 2:
+        lg[1] = 0xFF80  # no candidate: index 0
+        lg[2, 0] = 0x7FC0  # NaN at the scan's starting index
+    temps = np.array([0.0, 0.0, 0.9, 1.7, 0.4][:S], np.float32)
+    seed = torch.tensor([1234567], dtype=torch.int64, device="cuda")
+    out = torch.full((S,), -5, dtype=torch.int32, device="cuda")
+    ld, td = up(lg), up(temps)
+    for t, tdev in ((temps, td), (np.zeros_like(temps), torch.zeros_like(td))):
+        for _ in range(3):
+            lib().hip_sample(out.data_ptr(), ld.data_ptr(), tdev.data_ptr(), seed.data_ptr(), S, V, None)
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(out.cpu().numpy(), O.sample(lg, t, seed=1234567))
