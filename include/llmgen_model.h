@@ -1,9 +1,8 @@
 /*
  * llmgen_model.h -- C-ABI of the non-attention ops the Qwen3 forward needs around the attention path, in
- * libllmgen_attn.so.  They exist for the end-to-end greedy-token check, not as tuned kernels: each one computes
- * every output value in the same order and with the same roundings as the reference CPU backend
- * (the src/backend/cpu/ ops), so that a forward built from them differs from the CPU backend's only through the
- * attention kernels.  Each entry point replaces one extern of the reference CUDA backend with the same argument
+ * libllmgen_attn.so.  Each one computes every output value in the same order and with the same roundings as the
+ * reference CPU backend (the src/backend/cpu/ ops), so that a forward built from them differs from the CPU backend's
+ * only through the attention kernels.  Each entry point replaces one extern of the reference CUDA backend with the same argument
  * list (citations relative to the reference repository root):
  *   hip_embedding    src/backend/cuda/embedding/embedding.zig:7      (CPU: src/backend/cpu/embedding.zig)
  *   hip_rmsnorm      src/backend/cuda/norm/norm.zig:5                 (CPU: src/backend/cpu/norm.zig:57-89)
@@ -40,6 +39,15 @@ void hip_rmsnorm(uint16_t *out, const uint16_t *x, const float *w, long rows, in
  * y_f32 != 0, f32.  K % 8 == 0. */
 void hip_linear(void *y, int y_f32, const uint16_t *x, const uint16_t *w, int M, int N, int K);
 
+/* The products of one x with up to three weight matrices (q, k and v; gate and up) in one launch: yi [M, Ni] bf16 =
+ * x * wi [Ni, K]^T, each bit-identical to hip_linear.  Ni <= 0: no such product.  No reference extern. */
+void hip_linear3(uint16_t *y0, const uint16_t *w0, int N0, uint16_t *y1, const uint16_t *w1, int N1, uint16_t *y2,
+                 const uint16_t *w2, int N2, const uint16_t *x, int M, int K);
+
+/* y [M, N] bf16 = res [M, N] + x * w^T, bit-identical to hip_linear followed by hip_add (y may be res).  No reference
+ * extern. */
+void hip_linear_add(uint16_t *y, const uint16_t *res, const uint16_t *x, const uint16_t *w, int M, int N, int K);
+
 /* NEOX rotary embedding, in place allowed: for i < hd/2, out[i] = x[i]*cos[p][i] - x[i+hd/2]*sin[p][i] and
  * out[i+hd/2] = x[i+hd/2]*cos[p][i] + x[i]*sin[p][i], p = positions[t]; tables [max_seq, hd] f32.  hd even. */
 void hip_rope(uint16_t *out, const uint16_t *x, const float *cos_tab, const float *sin_tab, const int32_t *positions,
@@ -49,6 +57,9 @@ void hip_rope(uint16_t *out, const uint16_t *x, const float *cos_tab, const floa
 void hip_silu(uint16_t *out, const uint16_t *x, size_t n);
 void hip_add(uint16_t *out, const uint16_t *a, const uint16_t *b, size_t n);
 void hip_mul(uint16_t *out, const uint16_t *a, const uint16_t *b, size_t n);
+
+/* silu(gate) * up, bit-identical to hip_silu followed by hip_mul (out may be either input).  No reference extern. */
+void hip_silu_mul(uint16_t *out, const uint16_t *gate, const uint16_t *up, size_t n);
 
 /* out [S, H] bf16 = x[idx[s]] (gather_last).  H % 8 == 0. */
 void hip_gather_rows(uint16_t *out, const uint16_t *x, const int32_t *idx, int S, int H);

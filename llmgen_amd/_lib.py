@@ -58,10 +58,13 @@ SIGNATURES = {
     "hip_embedding": (None, [_P, _P, _P, _I, _I]),
     "hip_rmsnorm": (None, [_P, _P, _P, _L, _I, _F]),
     "hip_linear": (None, [_P, _I, _P, _P, _I, _I, _I]),
+    "hip_linear3": (None, [_P, _P, _I, _P, _P, _I, _P, _P, _I, _P, _I, _I]),
+    "hip_linear_add": (None, [_P, _P, _P, _P, _I, _I, _I]),
     "hip_rope": (None, [_P, _P, _P, _P, _P, _I, _I, _I]),
     "hip_silu": (None, [_P, _P, _SZ]),
     "hip_add": (None, [_P, _P, _P, _SZ]),
     "hip_mul": (None, [_P, _P, _P, _SZ]),
+    "hip_silu_mul": (None, [_P, _P, _P, _SZ]),
     "hip_gather_rows": (None, [_P, _P, _P, _I, _I]),
     "hip_sample": (None, [_P, _P, _P, _P, _I, _I, _P]),
     "hip_sample_scratch_bytes": (_SZ, [_I]),

@@ -26,7 +26,9 @@
 // 27 us; before, one output per lane with 256-column workgroups: 400 us).
 #include "hip_common.h"
 
+#include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #pragma clang fp contract(off)
 
@@ -42,11 +44,64 @@ __device__ __forceinline__ bool lin_half_ok(uint32_t h, uint32_t bias) {
     return (h & 0x7fffu) == 0 || (((h & 0x7fffu) + (bias & 0x7fffu)) & 0xC000u) == 0x4000u;
 }
 
-struct LinArgs {
+// One launch computes up to three products of the same x (q, k and v; gate and up): their column tiles follow each
+// other in the grid, a tile lies in one of them.  With `res`, y = res + (the product rounded to bf16), rounded again:
+// what a separate add of the stored product gives.
+struct LinOut {
     void *y;
-    const bf16_t *x, *w;
-    int M, N, K, y_f32, vec_out, tiles_m, tiles_n;
+    const bf16_t *w;
+    int N;
 };
+struct LinArgs {
+    LinOut out[3];
+    const bf16_t *x, *res;
+    int M, K, y_f32, vec_out, tiles_m;
+};
+// The product that column tile `tn` (tiles of TN columns) belongs to, and its first column there.
+__device__ __forceinline__ LinOut lin_out(const LinArgs &a, int tn, int TN, int &n0) {
+    LinOut o = a.out[0];
+    int first = (o.N + TN - 1) / TN;
+    if (tn >= first) {
+        tn -= first;
+        o = a.out[1];
+        first = (o.N + TN - 1) / TN;
+        if (tn >= first) {
+            tn -= first;
+            o = a.out[2];
+        }
+    }
+    n0 = tn * TN;
+    return o;
+}
+long lin_cols(const LinArgs &a, int TN) {
+    long t = 0;
+    for (const LinOut &o : a.out) t += (o.N + TN - 1) / TN;
+    return t;
+}
+__device__ __forceinline__ float lin_bf16(bf16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
+__device__ __forceinline__ float lin_round(float f) {
+    return lin_bf16(__builtin_bit_cast(bf16_t, (__bf16)f));
+}
+__device__ __forceinline__ void lin_put(const LinArgs &a, const LinOut &out, int m, int n, float v) {
+    const long o = (long)m * out.N + n;
+    if (a.res) v = lin_bf16(a.res[o]) + lin_round(v);
+    if (a.y_f32)
+        static_cast<float *>(out.y)[o] = v;
+    else
+        static_cast<bf16_t *>(out.y)[o] = __builtin_bit_cast(bf16_t, (__bf16)v);
+}
+// One output as the reference computes it: separate multiplies and adds.
+__device__ __forceinline__ float lin_plain(const bf16_t *xr, const bf16_t *wr, int K) {
+    float s = 0.0f;
+    for (int k = 0; k < K; k += 8) {
+        float xv[8], wv[8];
+        unpack_bf16x8(ld16(xr + k), xv);
+        unpack_bf16x8(ld16(wr + k), wv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s = s + xv[e] * wv[e];
+    }
+    return s;
+}
 
 // A workgroup's tile: WM x WN waves of MT x NT blocks of 16 x 16 outputs, PW extra waves that only stage (0: every
 // wave stages), KC values of k per LDS chunk.
@@ -71,10 +126,12 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
     __shared__ __attribute__((aligned(16))) float lds[2][T::ROWS * T::STRIDE];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // tiles in order of columns, each XCD (block index mod 8) a contiguous range of them
-    const int tiles = a.tiles_m * a.tiles_n;
+    const int tiles = gridDim.x;
     const int per = tiles >> 3, rem = tiles & 7, xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
     const int tile = xcd * per + min(xcd, rem) + at;
-    const int n0 = tile / a.tiles_m * T::TN, m0 = tile % a.tiles_m * T::TM;
+    int n0;
+    const LinOut out = lin_out(a, tile / a.tiles_m, T::TN, n0);
+    const int m0 = tile % a.tiles_m * T::TM;
     const int K = a.K, full = K / KC, tail = K - full * KC;
 
     // ---- staging: raw bf16 rows -> f32 in LDS, each 16 k of a row as [k % 4][k / 4]
@@ -178,9 +235,9 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
             for (int s = 0; s < T::SLOTS; ++s) {
                 const int i = sid + s * T::STAGERS, row = min(i / T::UNITS, T::ROWS - 1), u = i % T::UNITS;
                 is_w[s] = row < T::TN;
-                const long r = is_w[s] ? min(n0 + row, a.N - 1) : min(m0 + row - T::TN, a.M - 1);
+                const long r = is_w[s] ? min(n0 + row, out.N - 1) : min(m0 + row - T::TN, a.M - 1);
                 koff[s] = u * 16;
-                src[s] = (is_w[s] ? a.w : a.x) + r * K + u * 16;
+                src[s] = (is_w[s] ? out.w : a.x) + r * K + u * 16;
                 dst[s] = row * T::STRIDE + u * 16;
             }
             if (full > 0) {
@@ -243,33 +300,15 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
         else
             run(std::true_type{}, std::false_type{});
     }
-    // D of the instruction: columns are rows of x, a lane's four values are consecutive columns of y
-    auto put = [&](int m, int n, float v) {
-        const long o = (long)m * a.N + n;
-        if (a.y_f32)
-            static_cast<float *>(a.y)[o] = v;
-        else
-            static_cast<bf16_t *>(a.y)[o] = __builtin_bit_cast(bf16_t, (__bf16)v);
-    };
-    if (__builtin_expect(__syncthreads_or((int)bad), 0)) {
-        // a value outside its window: the reference's separate multiplies and adds
+    if (__builtin_expect(__syncthreads_or((int)bad), 0)) {  // a value outside its window
         for (int i = tid; i < T::TM * T::TN; i += T::THREADS) {
             const int m = m0 + i / T::TN, n = n0 + i % T::TN;
-            if (m >= a.M || n >= a.N) continue;
-            const bf16_t *xr = a.x + (long)m * K, *wr = a.w + (long)n * K;
-            float s = 0.0f;
-            for (int k = 0; k < K; k += 8) {
-                float xv[8], wv[8];
-                unpack_bf16x8(ld16(xr + k), xv);
-                unpack_bf16x8(ld16(wr + k), wv);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) s = s + xv[e] * wv[e];
-            }
-            put(m, n, s);
+            if (m < a.M && n < out.N) lin_put(a, out, m, n, lin_plain(a.x + (long)m * K, out.w + (long)n * K, K));
         }
         return;
     }
     if (PW && wave >= T::WAVES) return;
+    // D of the instruction: its columns are rows of x, a lane's four values are consecutive columns of y
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
         const int row = m0 + (wm * MT + m) * 16 + (lane & 15);
@@ -277,16 +316,23 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
             const int col = n0 + (wn * NT + n) * 16 + (lane >> 4) * 4;
-            if (a.vec_out && col < a.N) {
-                const long o = (long)row * a.N + col;
-                if (a.y_f32)
-                    *reinterpret_cast<f32x4_t *>(static_cast<float *>(a.y) + o) = acc[m][n];
-                else
-                    *reinterpret_cast<u32x2_t *>(static_cast<bf16_t *>(a.y) + o) =
-                        u32x2_t{pack_bf16x2(acc[m][n][0], acc[m][n][1]), pack_bf16x2(acc[m][n][2], acc[m][n][3])};
+            f32x4_t v = acc[m][n];
+            if (a.vec_out && col < out.N) {
+                const long o = (long)row * out.N + col;
+                if (a.y_f32) {
+                    *reinterpret_cast<f32x4_t *>(static_cast<float *>(out.y) + o) = v;
+                    continue;
+                }
+                if (a.res) {
+                    const u32x2_t r = *reinterpret_cast<const u32x2_t *>(a.res + o);
+                    v = f32x4_t{bf16lo_to_f32(r[0]) + lin_round(v[0]), bf16hi_to_f32(r[0]) + lin_round(v[1]),
+                                bf16lo_to_f32(r[1]) + lin_round(v[2]), bf16hi_to_f32(r[1]) + lin_round(v[3])};
+                }
+                *reinterpret_cast<u32x2_t *>(static_cast<bf16_t *>(out.y) + o) =
+                    u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
             } else {
                 for (int r = 0; r < 4; ++r)
-                    if (col + r < a.N) put(row, col + r, acc[m][n][r]);
+                    if (col + r < out.N) lin_put(a, out, row, col + r, v[r]);
             }
         }
     }
@@ -296,8 +342,109 @@ template <int MT, int NT, int WM, int WN, int PW, int KC, int PF>
 void linear_launch(LinArgs a) {
     using T = LinTile<MT, NT, WM, WN, PW, KC>;
     a.tiles_m = (a.M + T::TM - 1) / T::TM;
-    a.tiles_n = (a.N + T::TN - 1) / T::TN;
-    linear_kernel<MT, NT, WM, WN, PW, KC, PF><<<a.tiles_m * a.tiles_n, T::THREADS, 0, g_llmgen_stream>>>(a);
+    linear_kernel<MT, NT, WM, WN, PW, KC, PF>
+        <<<(unsigned)(a.tiles_m * lin_cols(a, T::TN)), T::THREADS, 0, g_llmgen_stream>>>(a);
+}
+
+// Up to eight rows and many columns (the LM head of a small decode step): bound by the read of w.  No LDS and no
+// barriers: a wave owns 32 columns and all rows, a lane reads 16-byte pieces of its own row of w straight into
+// registers (both halves of the wave hold the same 32 columns at alternate pieces), three stages of 64 k ahead, and
+// v_mfma_f32_4x4x1_f32 takes them as they lie: BLGP picks the half that holds k, CBSZ / ABID the four-row block of x
+// that does, so that nothing is moved between lanes.  8 x 151936 x 1024: 78 -> 63.5 us, one row 75 -> 57.5 us (5.4 TB/s);
+// at 16 rows the tiles below are as fast (79 us).
+constexpr int STREAM_ROWS = 8, STREAM_COLS = 128, STREAM_KC = 64, STREAM_PF = 3;
+
+template <int... Ks>
+__device__ __forceinline__ f32x4_t stream_products(f32x4_t acc, const float (&wf)[4][8], const float (&xf)[8],
+                                                   std::integer_sequence<int, Ks...>) {
+    // k of the stage, ascending: piece k / 8 of the row of w (wave half k / 8 % 2), block k / 8 of x, value k % 8
+    ((acc = __builtin_amdgcn_mfma_f32_4x4x1f32(xf[Ks % 8], wf[Ks / 16][Ks % 8], acc, 3, Ks / 8, 1 + (Ks / 8 & 1))), ...);
+    return acc;
+}
+
+__global__ void __launch_bounds__(256) linear_stream_kernel(const LinArgs a) {
+    constexpr int KC = STREAM_KC, PF = STREAM_PF;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int b0;
+    const LinOut out = lin_out(a, blockIdx.x, STREAM_COLS, b0);
+    const int n0 = b0 + wave * 32, K = a.K, full = K / KC, tail = K - full * KC;
+    const int half = lane >> 5, xpiece = (lane >> 2) & 7;
+    const bf16_t *wp = out.w + (long)min(n0 + (lane & 31), out.N - 1) * K + half * 8;
+    const bf16_t *xp = a.x + (long)min(half * 4 + (lane & 3), a.M - 1) * K + xpiece * 8;
+    u32x4_t wr[PF][4], xr[PF];
+    auto load = [&](int set, int c) {  // past the last full stage: that stage again
+        const long o = (long)min(c, full - 1) * KC;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) wr[set][i] = ld16(wp + o + i * 16);
+        xr[set] = ld16(xp + o);
+    };
+    auto load_tail = [&](int set) {
+        const long o = (long)full * KC;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            wr[set][i] = u32x4_t{0u, 0u, 0u, 0u};
+            if (i * 16 + half * 8 < tail) wr[set][i] = ld16(wp + o + i * 16);
+        }
+        xr[set] = u32x4_t{0u, 0u, 0u, 0u};
+        if (xpiece * 8 < tail) xr[set] = ld16(xp + o);
+    };
+    uint32_t bad = 0;
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    auto use = [&](int set) {
+        float wf[4][8], xf[8];
+        uint32_t in = LIN_IN;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            unpack_bf16x8(wr[set][i], wf[i]);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) in &= wr[set][i][d] + LIN_W_BIAS;
+        }
+        unpack_bf16x8(xr[set], xf);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) in &= xr[set][d] + LIN_X_BIAS;
+        if (__builtin_expect(__ballot(in != LIN_IN) != 0, 0)) {
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    bad |= !(lin_half_ok(wr[set][i][d] & 0xffffu, LIN_W_BIAS) &&
+                             lin_half_ok(wr[set][i][d] >> 16, LIN_W_BIAS));
+                bad |= !(lin_half_ok(xr[set][d] & 0xffffu, LIN_X_BIAS) && lin_half_ok(xr[set][d] >> 16, LIN_X_BIAS));
+            }
+        }
+        // the VALU work stays in one piece: each change between it and the matrix cores costs 8 cycles
+        __builtin_amdgcn_sched_barrier(0);
+        acc = stream_products(acc, wf, xf, std::make_integer_sequence<int, KC>{});
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int c = 0;
+    if (full > 0) {
+#pragma unroll
+        for (int p = 0; p < PF; ++p) load(p, p);
+        for (; c + PF <= full; c += PF)
+#pragma unroll
+            for (int p = 0; p < PF; ++p) {
+                use(p);
+                load(p, c + p + PF);
+            }
+    }
+#pragma unroll
+    for (int p = 0; p < PF; ++p) {
+        if (c + p == full && tail) load_tail(p);
+        if (c + p < full + (tail > 0)) use(p);
+    }
+    if (__builtin_expect(__syncthreads_or((int)bad), 0)) {  // a value outside its window
+        for (int i = threadIdx.x; i < a.M * STREAM_COLS; i += 256) {
+            const int m = i / STREAM_COLS, n = b0 + i % STREAM_COLS;
+            if (n < out.N) lin_put(a, out, m, n, lin_plain(a.x + (long)m * K, out.w + (long)n * K, K));
+        }
+        return;
+    }
+    const int n = n0 + (lane & 31);
+    if (n >= out.N) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        if (half * 4 + r < a.M) lin_put(a, out, half * 4 + r, n, acc[r]);
 }
 
 // Tiles of the throughput-bound sizes.  A launch takes about as long as the CU with the most tiles:
@@ -319,35 +466,61 @@ const LinChoice LIN_CHOICES[] = {{32, 32, 0.64f, linear_launch<1, 1, 2, 2, 0, 64
                                  {128, 128, 0.81f, linear_launch<4, 2, 2, 4, 0, 32, 2>}};
 
 void linear_dispatch(const LinArgs &a) {
-    const long blocks = (long)((a.M + 15) / 16) * ((a.N + 15) / 16);
+    const long cols = lin_cols(a, 16), blocks = (long)((a.M + 15) / 16) * cols;
     const int cus = llmgen_num_cus();
     // At most one 16 x 16 block per CU: one block and three staging waves a workgroup (8.2 us at 1 x 1024 x 1024,
     // 17.7 us at 32 x 1024 x 3072; two blocks and two staging waves 9.8 and 24 us).  At most two: two blocks and two
     // staging waves (11.3 us at 32 x 3072 x 1024; single blocks 12.6 us).
     if (blocks <= cus) return linear_launch<1, 1, 1, 1, 3, 128, 2>(a);
     if (blocks <= 2 * cus) return linear_launch<1, 1, 1, 2, 2, 64, 4>(a);
-    // Up to 16 rows and many columns: bound by the read of w; small workgroups, eight of them a CU (8 x 151936 x
-    // 1024: 78 us; 32 x 32 tiles, half of them empty, 108 us).
+    if (a.M <= STREAM_ROWS) {
+        linear_stream_kernel<<<(unsigned)lin_cols(a, STREAM_COLS), 256, 0, g_llmgen_stream>>>(a);
+        return;
+    }
+    // Up to 16 rows: small workgroups, eight of them a CU (16 x 151936 x 1024: 79 us; 32 x 32 tiles, half of them empty,
+    // 107 us).
     if (a.M <= 16) return linear_launch<1, 1, 1, 2, 0, 64, 2>(a);
     const LinChoice *best = nullptr;
     float cost = 0.f;
     for (const LinChoice &c : LIN_CHOICES) {
-        const long tiles = (long)((a.M + c.tm - 1) / c.tm) * ((a.N + c.tn - 1) / c.tn);
+        const long tiles = (long)((a.M + c.tm - 1) / c.tm) * lin_cols(a, c.tn);
         const float t = (float)((tiles + cus - 1) / cus) * (float)(c.tm * c.tn) / c.rate;
         if (!best || t < cost) best = &c, cost = t;
     }
     best->launch(a);
 }
 
+bool lin_reject(const char *what) {
+    fprintf(stderr, "llmgen: %s: K must be a positive multiple of 8\n", what);
+    return true;
+}
+// whether four outputs of a row can be moved as one word
+bool lin_words(const void *p, int N, int bytes) { return N % 4 == 0 && (uintptr_t)p % (4 * bytes) == 0; }
+
 }  // namespace
 
-extern "C" void hip_linear(void *y, int y_f32, const uint16_t *x, const uint16_t *w, int M, int N, int K) {
+extern "C" {
+
+void hip_linear(void *y, int y_f32, const uint16_t *x, const uint16_t *w, int M, int N, int K) {
     if (M <= 0 || N <= 0) return;
-    if (K <= 0 || K % 8 != 0) {
-        fprintf(stderr, "llmgen: hip_linear: K must be a positive multiple of 8\n");
-        return;
-    }
-    // four outputs of a row are stored as one word where each such group is aligned for it
-    const int vec = N % 4 == 0 && (uintptr_t)y % (y_f32 ? 16 : 8) == 0;
-    linear_dispatch(LinArgs{y, x, w, M, N, K, y_f32, vec, 0, 0});
+    if ((K <= 0 || K % 8 != 0) && lin_reject("hip_linear")) return;
+    linear_dispatch(LinArgs{{{y, w, N}, {}, {}}, x, nullptr, M, K, y_f32, lin_words(y, N, y_f32 ? 4 : 2), 0});
 }
+
+void hip_linear_add(uint16_t *y, const uint16_t *res, const uint16_t *x, const uint16_t *w, int M, int N, int K) {
+    if (M <= 0 || N <= 0) return;
+    if ((K <= 0 || K % 8 != 0) && lin_reject("hip_linear_add")) return;
+    const int vec = lin_words(y, N, 2) && lin_words(res, N, 2);
+    linear_dispatch(LinArgs{{{y, w, N}, {}, {}}, x, res, M, K, 0, vec, 0});
+}
+
+void hip_linear3(uint16_t *y0, const uint16_t *w0, int N0, uint16_t *y1, const uint16_t *w1, int N1, uint16_t *y2,
+                 const uint16_t *w2, int N2, const uint16_t *x, int M, int K) {
+    N0 = std::max(N0, 0), N1 = std::max(N1, 0), N2 = std::max(N2, 0);
+    if (M <= 0 || (N0 | N1 | N2) == 0) return;
+    if ((K <= 0 || K % 8 != 0) && lin_reject("hip_linear3")) return;
+    const int vec = lin_words(y0, N0, 2) && lin_words(y1, N1, 2) && lin_words(y2, N2, 2);
+    linear_dispatch(LinArgs{{{y0, w0, N0}, {y1, w1, N1}, {y2, w2, N2}}, x, nullptr, M, K, 0, vec, 0});
+}
+
+}  // extern "C"

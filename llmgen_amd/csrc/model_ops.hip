@@ -115,6 +115,9 @@ struct SiluOp {
 struct AddOp {
     __device__ __forceinline__ float operator()(float a, float b) const { return a + b; }
 };
+struct SiluMulOp {  // SiLU's result is rounded to bf16 before the product, as when it is stored in between
+    __device__ __forceinline__ float operator()(float v, float u) const { return bf2f(f2bf(SiluOp{}(v, 0.f))) * u; }
+};
 struct MulOp {
     __device__ __forceinline__ float operator()(float a, float b) const { return a * b; }
 };
@@ -359,6 +362,10 @@ void hip_silu(uint16_t *out, const uint16_t *x, size_t n) { elementwise(out, x, 
 void hip_add(uint16_t *out, const uint16_t *a, const uint16_t *b, size_t n) { elementwise(out, a, b, n, AddOp{}); }
 
 void hip_mul(uint16_t *out, const uint16_t *a, const uint16_t *b, size_t n) { elementwise(out, a, b, n, MulOp{}); }
+
+void hip_silu_mul(uint16_t *out, const uint16_t *gate, const uint16_t *up, size_t n) {
+    elementwise(out, gate, up, n, SiluMulOp{});
+}
 
 void hip_gather_rows(uint16_t *out, const uint16_t *x, const int32_t *idx, int S, int H) {
     if (S <= 0) return;

@@ -179,9 +179,11 @@ class Qwen3:
                 fused_qk: bool = True) -> List[int]:
         """One step: entries[i] computes positions [q_start, q_start + q_len) of sequence i with this step's
         token ids (concatenated in entry order).  ``temps[i]`` > 0 samples sequence i (Gumbel-max), else greedy.
-        ``seed`` resets the step-seed state (executor.zig:773 advances it every step).  ``fused_qk`` runs q/k norm
-        + RoPE + the KV write as one kernel (hip_qk_norm_rope_store_kv); the unfused path runs the reference
-        graph's five launches.  Both give identical values."""
+        ``seed`` resets the step-seed state (executor.zig:773 advances it every step).  ``fused_qk`` runs a
+        layer in nine launches: the projections of one input together (hip_linear3), q/k norm + RoPE + the KV write
+        as one kernel (hip_qk_norm_rope_store_kv), the residual adds with the product before them (hip_linear_add)
+        and SiLU with the product after it (hip_silu_mul); without it the reference graph's launches run one by one.
+        Both give identical values."""
         cfg, L = self.cfg, self.L
         T, S = sum(e.q_len for e in entries), len(entries)
         if len(ids) != T or T > self.max_tokens or S > self.max_seqs:
@@ -224,30 +226,38 @@ class Qwen3:
         for i in range(cfg.n_layers):
             b = f"blk.{i}."
             L.hip_rmsnorm(p(xn), p(x), p(W[b + "attn_norm.weight"]), T, H, cfg.rms_eps)
-            L.hip_linear(p(q), 0, p(xn), p(W[b + "attn_q.weight"]), T, nq * hd, H)
-            L.hip_linear(p(k), 0, p(xn), p(W[b + "attn_k.weight"]), T, nkv * hd, H)
-            L.hip_linear(p(v), 0, p(xn), p(W[b + "attn_v.weight"]), T, nkv * hd, H)
+            w = lambda n: W[b + n + ".weight"].data_ptr()  # noqa: E731,B023
             kv = self.kv[i]
             if fused_qk:
-                L.hip_qk_norm_rope_store_kv(p(q), p(kv.k), p(kv.v), p(q), p(k), p(v),
-                                            p(W[b + "attn_q_norm.weight"]), p(W[b + "attn_k_norm.weight"]),
-                                            cfg.rms_eps, p(self.cos), p(self.sin), g.pos, g.slots, T, nq, nkv, hd,
-                                            cfg.block_size)
+                L.hip_linear3(p(q), w("attn_q"), nq * hd, p(k), w("attn_k"), nkv * hd, p(v), w("attn_v"), nkv * hd,
+                              p(xn), T, H)
+                L.hip_qk_norm_rope_store_kv(p(q), p(kv.k), p(kv.v), p(q), p(k), p(v), w("attn_q_norm"),
+                                            w("attn_k_norm"), cfg.rms_eps, p(self.cos), p(self.sin), g.pos, g.slots,
+                                            T, nq, nkv, hd, cfg.block_size)
+                Hx.paged_attention(g, attn, q, k, v, kv.k, kv.v, store_kv=False)
+                L.hip_linear_add(p(x), p(x), p(attn), w("attn_output"), T, H, nq * hd)
+                L.hip_rmsnorm(p(xn), p(x), w("ffn_norm"), T, H, cfg.rms_eps)
+                L.hip_linear3(p(gate), w("ffn_gate"), F, p(up), w("ffn_up"), F, None, None, 0, p(xn), T, H)
+                L.hip_silu_mul(p(gate), p(gate), p(up), T * F)
+                L.hip_linear_add(p(x), p(x), p(gate), w("ffn_down"), T, H, F)
             else:
-                L.hip_rmsnorm(p(q), p(q), p(W[b + "attn_q_norm.weight"]), T * nq, hd, cfg.rms_eps)
-                L.hip_rmsnorm(p(k), p(k), p(W[b + "attn_k_norm.weight"]), T * nkv, hd, cfg.rms_eps)
+                L.hip_linear(p(q), 0, p(xn), w("attn_q"), T, nq * hd, H)
+                L.hip_linear(p(k), 0, p(xn), w("attn_k"), T, nkv * hd, H)
+                L.hip_linear(p(v), 0, p(xn), w("attn_v"), T, nkv * hd, H)
+                L.hip_rmsnorm(p(q), p(q), w("attn_q_norm"), T * nq, hd, cfg.rms_eps)
+                L.hip_rmsnorm(p(k), p(k), w("attn_k_norm"), T * nkv, hd, cfg.rms_eps)
                 L.hip_rope(p(q), p(q), p(self.cos), p(self.sin), g.pos, T, nq, hd)
                 L.hip_rope(p(k), p(k), p(self.cos), p(self.sin), g.pos, T, nkv, hd)
-            Hx.paged_attention(g, attn, q, k, v, kv.k, kv.v, store_kv=not fused_qk)
-            L.hip_linear(p(o), 0, p(attn), p(W[b + "attn_output.weight"]), T, H, nq * hd)
-            L.hip_add(p(x), p(x), p(o), T * H)
-            L.hip_rmsnorm(p(xn), p(x), p(W[b + "ffn_norm.weight"]), T, H, cfg.rms_eps)
-            L.hip_linear(p(gate), 0, p(xn), p(W[b + "ffn_gate.weight"]), T, F, H)
-            L.hip_linear(p(up), 0, p(xn), p(W[b + "ffn_up.weight"]), T, F, H)
-            L.hip_silu(p(gate), p(gate), T * F)
-            L.hip_mul(p(gate), p(gate), p(up), T * F)
-            L.hip_linear(p(o), 0, p(gate), p(W[b + "ffn_down.weight"]), T, H, F)
-            L.hip_add(p(x), p(x), p(o), T * H)
+                Hx.paged_attention(g, attn, q, k, v, kv.k, kv.v)
+                L.hip_linear(p(o), 0, p(attn), w("attn_output"), T, H, nq * hd)
+                L.hip_add(p(x), p(x), p(o), T * H)
+                L.hip_rmsnorm(p(xn), p(x), w("ffn_norm"), T, H, cfg.rms_eps)
+                L.hip_linear(p(gate), 0, p(xn), w("ffn_gate"), T, F, H)
+                L.hip_linear(p(up), 0, p(xn), w("ffn_up"), T, F, H)
+                L.hip_silu(p(gate), p(gate), T * F)
+                L.hip_mul(p(gate), p(gate), p(up), T * F)
+                L.hip_linear(p(o), 0, p(gate), w("ffn_down"), T, H, F)
+                L.hip_add(p(x), p(x), p(o), T * H)
         L.hip_rmsnorm(p(xn), p(x), p(W["output_norm.weight"]), T, H, cfg.rms_eps)
         last = self._empty(S, H)
         L.hip_gather_rows(p(last), p(xn), g.last, S, H)

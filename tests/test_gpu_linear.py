@@ -41,10 +41,11 @@ def draw(rng, *shape, std=1.0):
     return O.f32_to_bf16((std * rng.standard_normal(shape)).astype(np.float32))
 
 
-# (M, N, K): one 16 x 16 block a workgroup, two blocks, up to 16 rows of many columns, then 32 x 32, 64 x 64, 64 x 192,
+# (M, N, K): one 16 x 16 block a workgroup, two blocks, up to 16 and up to 8 rows of many columns, then 32 x 32, 64 x 64, 64 x 192,
 # 96 x 192 and 128 x 128 tiles
 @pytest.mark.parametrize("M,N,K", [(1, 1, 8), (1, 16, 128), (17, 100, 24), (16, 1024, 1000), (3, 2049, 264),
-                                   (33, 1700, 72), (40, 2000, 320), (16, 8200, 40), (5, 9001, 200), (50, 3000, 200),
+                                   (33, 1700, 72), (40, 2000, 320), (16, 8200, 40), (5, 9001, 200),
+                                   (8, 8196, 8), (1, 8321, 64), (8, 8200, 328), (50, 3000, 200),
                                    (129, 1031, 64), (512, 2048, 72), (1000, 3060, 40), (2051, 2048, 24),
                                    (2048, 6144, 16)])
 def test_linear_tiles_bit_exact(gpu, M, N, K):
@@ -59,7 +60,7 @@ def test_linear_any_output_alignment(gpu, N, offset, y_f32):
     check(draw(rng, 19, 48), draw(rng, N, 48), y_f32, offset)
 
 
-@pytest.mark.parametrize("M,N,K", [(9, 70, 136), (40, 2000, 72), (12, 8300, 72), (200, 1100, 200), (512, 2048, 40)])
+@pytest.mark.parametrize("M,N,K", [(9, 70, 136), (40, 2000, 72), (12, 8300, 72), (7, 8300, 136), (200, 1100, 200), (512, 2048, 40)])
 @pytest.mark.parametrize("what", ["zeros", "tiny", "huge", "nonfinite", "edges"])
 def test_linear_values_outside_the_exact_window(gpu, M, N, K, what):
     """Zeros stay on the fast path; values whose products leave f32's exact range (or are not finite) must take the
@@ -81,3 +82,41 @@ def test_linear_values_outside_the_exact_window(gpu, M, N, K, what):
         w[N // 2] = rng.choice(np.array(special, np.uint16), K)
     check(x, w, y_f32=True)
     check(x, w, y_f32=False)
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 33, 300])
+@pytest.mark.parametrize("Ns", [(2048, 1024, 1024), (3000, 3001, 0), (40, 24, 7), (0, 100, 33)])
+def test_linear3_equals_single_products(gpu, M, Ns):
+    """Column tiles of the three products share a grid: each must stay within its own matrix and output."""
+    K, rng = 72, np.random.default_rng(M + sum(Ns))
+    x, ws = draw(rng, M, K), [draw(rng, max(n, 1), K, std=0.1) for n in Ns]
+    ws[1][0, 0] = 0x7F80  # only tiles of the second product take the separate operations
+    xd, wd = torch.from_numpy(x.view(np.int16)).cuda(), [torch.from_numpy(w.view(np.int16)).cuda() for w in ws]
+    ys = [torch.full((M * n + 8,), 77, dtype=torch.int16, device="cuda") for n in Ns]
+    args = [a for y, w, n in zip(ys, wd, Ns) for a in ((y.data_ptr(), w.data_ptr(), n) if n else (None, None, 0))]
+    lib().hip_linear3(*args, xd.data_ptr(), M, K)
+    torch.cuda.synchronize()
+    assert lib().hip_last_error() == 0
+    for y, w, n in zip(ys, ws, Ns):
+        got, ref = y.cpu().numpy(), run(x, w, False)[:, :n] if n else np.zeros((M, 0), np.uint16)
+        assert (got[M * n:] == 77).all()
+        np.testing.assert_array_equal(got[:M * n].view(np.uint16).reshape(M, n), ref)
+
+
+@pytest.mark.parametrize("M,N", [(1, 1024), (8, 8300), (12, 8300), (33, 1701), (300, 1024)])
+@pytest.mark.parametrize("what", ["in_place", "unaligned", "outside"])
+def test_linear_add_equals_linear_then_add(gpu, M, N, what):
+    K, rng = 136, np.random.default_rng(M + N)
+    x, w, res = draw(rng, M, K), draw(rng, N, K, std=0.1), draw(rng, M, N)
+    if what == "outside":
+        x[0, 3] = 0x0001
+    shift = 1 if what == "unaligned" else 0
+    xd, wd = (torch.from_numpy(a.view(np.int16)).cuda() for a in (x, w))
+    rd = torch.zeros(M * N + 1, dtype=torch.int16, device="cuda")
+    rd[shift:shift + M * N] = torch.from_numpy(res.view(np.int16).reshape(-1)).cuda()
+    yd = rd if what == "in_place" else torch.zeros(M * N, dtype=torch.int16, device="cuda")
+    lib().hip_linear_add(yd.data_ptr(), rd.data_ptr() + 2 * shift, xd.data_ptr(), wd.data_ptr(), M, N, K)
+    torch.cuda.synchronize()
+    assert lib().hip_last_error() == 0
+    got = yd.cpu().numpy()[:M * N].view(np.uint16).reshape(M, N)
+    np.testing.assert_array_equal(got, O.add(res.reshape(-1), O.linear(x, w).reshape(-1)).reshape(M, N))

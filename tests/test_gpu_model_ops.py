@@ -56,6 +56,16 @@ def test_elementwise_tails_and_alignment(gpu, n, offset):
         assert not got[n:].any()
 
 
+def test_silu_mul_equals_silu_then_mul(gpu):
+    rng = np.random.default_rng(3)
+    a, b = up(draw(rng, 3077, std=4.0)), up(draw(rng, 3077))
+    ref, out = torch.empty_like(a), a.clone()
+    lib().hip_silu(ref.data_ptr(), a.data_ptr(), a.numel())
+    lib().hip_mul(ref.data_ptr(), ref.data_ptr(), b.data_ptr(), a.numel())
+    lib().hip_silu_mul(out.data_ptr(), out.data_ptr(), b.data_ptr(), a.numel())
+    np.testing.assert_array_equal(down(out), down(ref))
+
+
 def test_silu_every_value(gpu):
     """All 65536 inputs against x / (1 + exp(-x)) with exp rounded once to f32, as a correctly rounded expf gives it."""
     bits = np.arange(65536, dtype=np.uint32).astype(np.uint16)
