@@ -22,8 +22,8 @@
 //
 // Small steps (decode) are bound by the chain of one output instead: 8 cycles per k, 3.4 us at K = 1024.  There a
 // wave owns a single 16 x 16 tile and staging is left to producer waves of the same workgroup, which sit on the other
-// SIMDs, so the chain's SIMD does nothing else (K = 3072, N = 1024, 32 rows: 17 us; with the staging in the same wave
-// 27 us; before, one output per lane with 256-column workgroups: 400 us).
+// SIMDs, so the chain's SIMD does nothing else (K = 3072, N = 1024, 32 rows: 17.3 us; with the staging in the same wave
+// 26 us; one output per lane with 256-column workgroups, as multiplies and adds: 400 us).
 #include "hip_common.h"
 
 #include <algorithm>
@@ -103,6 +103,27 @@ __device__ __forceinline__ float lin_plain(const bf16_t *xr, const bf16_t *wr, i
     return s;
 }
 
+// The order of one step's instructions: the LDS reads spread between the matrix instructions, then the staging's VALU
+// work in one piece, then its LDS writes spread likewise.  A wave issues in order and its LDS queue is short, so reads
+// or writes issued together hold up the matrix instructions behind them, and every change between VALU and matrix
+// instructions costs 8 cycles (as the compiler orders a step by itself: 997 x 1024 x 3072 70.9 us, so 56.5 us).
+template <int READS, int WRITES, int PRODUCTS>
+__device__ __forceinline__ void lin_interleave() {
+    constexpr int PER = PRODUCTS / (READS + WRITES) > 0 ? PRODUCTS / (READS + WRITES) : 1;
+#pragma unroll
+    for (int i = 0; i < READS; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);  // matrix instructions
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);    // LDS read
+    }
+    if (WRITES) __builtin_amdgcn_sched_group_barrier(0x002, 64, 0);  // VALU
+#pragma unroll
+    for (int i = 0; i < WRITES; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
+        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, PRODUCTS, 0);
+}
+
 // A workgroup's tile: WM x WN waves of MT x NT blocks of 16 x 16 outputs, PW extra waves that only stage (0: every
 // wave stages), KC values of k per LDS chunk.
 template <int MT, int NT, int WM, int WN, int PW, int KC>
@@ -163,7 +184,7 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
                 if (T::has(sid, s) && koff[s] + h * 8 < tail) r[s][h] = ld16(src[s] + base + h * 8);
             }
     };
-    auto stage = [&](const u32x4_t (&r)[T::SLOTS][2], int buf) {
+    auto stage_put = [&](const u32x4_t (&r)[T::SLOTS][2], int buf) {
         uint32_t in = LIN_IN;
 #pragma unroll
         for (int s = 0; s < T::SLOTS; ++s) {
@@ -180,6 +201,9 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
             for (int q = 0; q < 4; ++q)
                 *reinterpret_cast<f32x4_t *>(&lds[buf][dst[s] + q * 4]) = f32x4_t{f[q], f[4 + q], f[8 + q], f[12 + q]};
         }
+        return in;
+    };
+    auto stage_check = [&](const u32x4_t (&r)[T::SLOTS][2], uint32_t in) {
         if (__builtin_expect(__ballot(in != LIN_IN) != 0, 0)) {
 #pragma unroll
             for (int s = 0; s < T::SLOTS; ++s) {
@@ -193,6 +217,7 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
             }
         }
     };
+    auto stage = [&](const u32x4_t (&r)[T::SLOTS][2], int buf) { stage_check(r, stage_put(r, buf)); };
 
     // ---- products
     const int wm = wave % WM, wn = wave / WM;
@@ -266,12 +291,19 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
         for (; i + PF + 2 <= full; i += PF) {
 #pragma unroll
             for (int p = 0; p < PF; ++p) {
+                uint32_t in = LIN_IN;
                 if constexpr (C) fetch((p + 1) & 1);
+                if constexpr (S) in = stage_put(raw[(p + 2) % PF], p & 1);
+                if constexpr (C) {
+                    compute(p & 1);
+                    // (a last slot of only some waves is a branch, and its own scheduling region)
+                    if constexpr (!S || T::WORK % T::STAGERS == 0)
+                        lin_interleave<T::UNITS *(MT + NT), S ? T::SLOTS * 4 : 0, T::UNITS * 4 * MT * NT>();
+                }
                 if constexpr (S) {
-                    stage(raw[(p + 2) % PF], p & 1);
+                    stage_check(raw[(p + 2) % PF], in);
                     load(raw[(p + 2) % PF]);
                 }
-                if constexpr (C) compute(p & 1);
                 __syncthreads();
             }
         }
@@ -449,37 +481,38 @@ __global__ void __launch_bounds__(256) linear_stream_kernel(const LinArgs a) {
 
 // Tiles of the throughput-bound sizes.  A launch takes about as long as the CU with the most tiles:
 // ceil(tiles / CUs) * blocks of a tile / rate, where `rate` is the share of the matrix cores' peak that the tile
-// reached on sizes it fits (launch time taken off): 0.64 for 32 x 32 (M = 2051, N = K = 1024: 50.8 us), 0.75 for
-// 64 x 64 (997 x 3072 x 1024: 58.2 us), 0.76 for 64 x 192 and 96 x 192 (57.4 us; 2051 x 2048 x 1024: 83.8 us) and
-// 0.81 for 128 x 128 (2048 x 6144 x 2048: 407 us = 127 TFLOP/s).  Larger tiles stage less per product but quantise
-// coarser; the best of the five by this rule was within 4 % of the best of 33 measured tiles on 12 sizes from
-// 200 x 3072 x 1024 to 3000 x 4096 x 2560.
+// reached on sizes it fits (launch time taken off): 0.70 for 32 x 32 (2051 x 1024 x 1024: 47.3 us; 631 x 1024 x 3072:
+// 47.8 us), 0.80 for 64 x 64 (997 x 1024 x 3072: 56.5 us), 0.83 for 64 x 192 (997 x 3072 x 1024: 53.6 us), 0.765 for
+// 96 x 192 (2051 x 2048 x 1024: 83.8 us) and 0.85 for 128 x 128 (2048 x 6144 x 2048: 385 us = 134 TFLOP/s).  Larger
+// tiles stage less per product but quantise coarser; over 14 sizes from 200 x 1024 x 1024 to 3000 x 4096 x 2560 the
+// choice was within 3 % of the best of 31 measured tiles.
 struct LinChoice {
     int tm, tn;
     float rate;
     void (*launch)(LinArgs);
 };
-const LinChoice LIN_CHOICES[] = {{32, 32, 0.64f, linear_launch<1, 1, 2, 2, 0, 64, 2>},
-                                 {64, 64, 0.75f, linear_launch<2, 2, 2, 2, 0, 32, 2>},
-                                 {64, 192, 0.76f, linear_launch<2, 3, 2, 4, 0, 32, 2>},
+const LinChoice LIN_CHOICES[] = {{32, 32, 0.70f, linear_launch<1, 1, 2, 2, 0, 64, 2>},
+                                 {64, 64, 0.80f, linear_launch<2, 2, 2, 2, 0, 32, 2>},
+                                 {64, 192, 0.83f, linear_launch<2, 3, 2, 4, 0, 32, 2>},
                                  {96, 192, 0.765f, linear_launch<3, 3, 2, 4, 0, 32, 2>},
-                                 {128, 128, 0.81f, linear_launch<4, 2, 2, 4, 0, 32, 2>}};
+                                 {128, 128, 0.85f, linear_launch<4, 2, 2, 4, 0, 32, 2>}};
 
 void linear_dispatch(const LinArgs &a) {
-    const long cols = lin_cols(a, 16), blocks = (long)((a.M + 15) / 16) * cols;
+    const long blocks = (long)((a.M + 15) / 16) * lin_cols(a, 16);
     const int cus = llmgen_num_cus();
-    // At most one 16 x 16 block per CU: one block and three staging waves a workgroup (8.2 us at 1 x 1024 x 1024,
-    // 17.7 us at 32 x 1024 x 3072; two blocks and two staging waves 9.8 and 24 us).  At most two: two blocks and two
-    // staging waves (11.3 us at 32 x 3072 x 1024; single blocks 12.6 us).
+    // At most one 16 x 16 block per CU: one block and three staging waves a workgroup (7.8 us at 1 x 1024 x 1024,
+    // 17.3 us at 32 x 1024 x 3072; 32 x 32 tiles 9.5 and 26 us).
     if (blocks <= cus) return linear_launch<1, 1, 1, 1, 3, 128, 2>(a);
+    // At most two: two blocks and two staging waves (11.2 us at 32 x 3072 x 1024, 12 us as single blocks; 32 x 32 tiles
+    // take 10.8 us back to back, but 0.5 us more between other kernels: an MLP of 32 tokens 48.2 us, so 46.8 us).
     if (blocks <= 2 * cus) return linear_launch<1, 1, 1, 2, 2, 64, 4>(a);
-    if (a.M <= STREAM_ROWS) {
+    // Up to 16 rows and more blocks: bound by the read of w.  To 8 rows the stream above, to 16 small
+    // workgroups, eight of them a CU (16 x 151936 x 1024: 79 us; 32 x 32 tiles, half of them empty, 107 us).
+    if (a.M <= 16) {
+        if (a.M > STREAM_ROWS) return linear_launch<1, 1, 1, 2, 0, 64, 2>(a);
         linear_stream_kernel<<<(unsigned)lin_cols(a, STREAM_COLS), 256, 0, g_llmgen_stream>>>(a);
         return;
     }
-    // Up to 16 rows: small workgroups, eight of them a CU (16 x 151936 x 1024: 79 us; 32 x 32 tiles, half of them empty,
-    // 107 us).
-    if (a.M <= 16) return linear_launch<1, 1, 1, 2, 0, 64, 2>(a);
     const LinChoice *best = nullptr;
     float cost = 0.f;
     for (const LinChoice &c : LIN_CHOICES) {
