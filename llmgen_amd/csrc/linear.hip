@@ -481,20 +481,20 @@ __global__ void __launch_bounds__(256) linear_stream_kernel(const LinArgs a) {
 
 // Tiles of the throughput-bound sizes.  A launch takes about as long as the CU with the most tiles:
 // ceil(tiles / CUs) * blocks of a tile / rate, where `rate` is the share of the matrix cores' peak that the tile
-// reached on sizes it fits (launch time taken off): 0.70 for 32 x 32 (2051 x 1024 x 1024: 47.3 us; 631 x 1024 x 3072:
-// 47.8 us), 0.80 for 64 x 64 (997 x 1024 x 3072: 56.5 us), 0.83 for 64 x 192 (997 x 3072 x 1024: 53.6 us), 0.765 for
-// 96 x 192 (2051 x 2048 x 1024: 83.8 us) and 0.85 for 128 x 128 (2048 x 6144 x 2048: 385 us = 134 TFLOP/s).  Larger
-// tiles stage less per product but quantise coarser; over 14 sizes from 200 x 1024 x 1024 to 3000 x 4096 x 2560 the
-// choice was within 3 % of the best of 31 measured tiles.
+// reached on sizes it fits (launch time taken off): 0.68 for 32 x 32 (631 x 1024 x 3072: 47.8 us; 350 x 1024 x 3072:
+// 34.4 us), 0.76 for 32 x 96 (2051 x 1024 x 1024: 43.2 us; 32 x 151936 x 1024: 102 us), 0.80 for 64 x 64 (997 x 1024 x
+// 3072: 56.5 us), 0.83 for 64 x 192 (997 x 3072 x 1024: 53.6 us) and 0.85 for 128 x 128 (2048 x 6144 x 2048: 385 us =
+// 134 TFLOP/s).  Larger tiles stage less per product but quantise coarser.  All five stage in whole slots per wave (a
+// slot that only some waves have splits the step's schedule: 96 x 32 with a 64-value chunk 10 % slower).
 struct LinChoice {
     int tm, tn;
     float rate;
     void (*launch)(LinArgs);
 };
-const LinChoice LIN_CHOICES[] = {{32, 32, 0.70f, linear_launch<1, 1, 2, 2, 0, 64, 2>},
+const LinChoice LIN_CHOICES[] = {{32, 32, 0.68f, linear_launch<1, 1, 2, 2, 0, 64, 2>},
+                                 {32, 96, 0.76f, linear_launch<1, 3, 2, 2, 0, 32, 2>},
                                  {64, 64, 0.80f, linear_launch<2, 2, 2, 2, 0, 32, 2>},
                                  {64, 192, 0.83f, linear_launch<2, 3, 2, 4, 0, 32, 2>},
-                                 {96, 192, 0.765f, linear_launch<3, 3, 2, 4, 0, 32, 2>},
                                  {128, 128, 0.85f, linear_launch<4, 2, 2, 4, 0, 32, 2>}};
 
 void linear_dispatch(const LinArgs &a) {

@@ -42,11 +42,11 @@ def draw(rng, *shape, std=1.0):
 
 
 # (M, N, K): one 16 x 16 block a workgroup, two blocks, up to 16 and up to 8 rows of many columns, then 32 x 32, 64 x 64, 64 x 192,
-# 96 x 192 and 128 x 128 tiles
+# 32 x 96 and 128 x 128 tiles
 @pytest.mark.parametrize("M,N,K", [(1, 1, 8), (1, 16, 128), (17, 100, 24), (16, 1024, 1000), (3, 2049, 264),
                                    (33, 1700, 72), (40, 2000, 320), (16, 8200, 40), (5, 9001, 200),
                                    (8, 8196, 8), (1, 8321, 64), (8, 8200, 328), (50, 3000, 200),
-                                   (129, 1031, 64), (512, 2048, 72), (1000, 3060, 40), (2051, 2048, 24),
+                                   (129, 1031, 64), (512, 2048, 72), (1000, 3060, 40), (2051, 2048, 24), (200, 3001, 104),
                                    (2048, 6144, 16)])
 def test_linear_tiles_bit_exact(gpu, M, N, K):
     rng = np.random.default_rng(M + 3 * N + K)
