@@ -36,7 +36,8 @@ __global__ void embedding_kernel(bf16_t *out, const int *ids, const bf16_t *w, i
 // lanes square the row's values (exactly what the reference adds, one rounded multiply each) and leave them in LDS,
 // and the chain is a run of adds fed by 16-byte LDS reads.  A wave owns R rows, 64 / R lanes each; every lane runs its
 // row's chain (the reads of a row's lanes are one broadcast address), so the sum needs no exchange afterwards.
-// Measured, D = 1024: 32 rows 16 -> 5.6 us, 2051 rows 38 -> 7.3 us (one lane of a wave forming each square and sum).
+// Measured, D = 1024: 32 rows 14.7 -> 5.2 us, 2051 rows 36 -> 7.4 us (before: one lane of a wave formed each square and
+// sum).
 constexpr int NORM_MAX_D = 8192;
 template <int R>
 __global__ void __launch_bounds__(64) rmsnorm_kernel(bf16_t *out, const bf16_t *x, const float *w, long rows, int D,
@@ -48,44 +49,92 @@ __global__ void __launch_bounds__(64) rmsnorm_kernel(bf16_t *out, const bf16_t *
     const bool valid = (long)blockIdx.x * R + threadIdx.x / L < rows;
     const bf16_t *xr = x + r * D;
     float *sr = sq + threadIdx.x / L * (D + 4);  // rows start in different banks
-#pragma unroll 4
-    for (int c = sub; c < chunks; c += L) {
+    // Few rows (one a wave) are bound by latencies: up to KEEP pieces of a row stay in registers, with their gains loaded
+    // before the chain, and the chain reads ahead (32 rows of 1024: 5.7 us without, 5.2 us with).  Many rows need the
+    // waves instead of the registers (8195 x 128 in this form 7.0 us, not 5.2).
+    constexpr int KEEP = R == 1 ? 4 : 1, AHEAD = R == 1 ? 2 : 1;
+    const bool kept = R == 1 && chunks <= KEEP * L;
+    u32x4_t raw[KEEP];
+    f32x4_t gain[KEEP][2];
+    auto square = [&](u32x4_t v, int c) {
         float f[8];
-        unpack_bf16x8(ld16(xr + c * 8), f);
+        unpack_bf16x8(v, f);
 #pragma unroll
         for (int h = 0; h < 2; ++h)
             *reinterpret_cast<f32x4_t *>(sr + c * 8 + h * 4) =
                 f32x4_t{f[4 * h] * f[4 * h], f[4 * h + 1] * f[4 * h + 1], f[4 * h + 2] * f[4 * h + 2],
                         f[4 * h + 3] * f[4 * h + 3]};
+    };
+    if (kept) {
+#pragma unroll
+        for (int i = 0; i < KEEP; ++i)
+            if (sub + i * L < chunks) raw[i] = ld16(xr + (sub + i * L) * 8);
+#pragma unroll
+        for (int i = 0; i < KEEP; ++i)
+            if (sub + i * L < chunks) {
+                gain[i][0] = *reinterpret_cast<const f32x4_t *>(w + (sub + i * L) * 8);
+                gain[i][1] = *reinterpret_cast<const f32x4_t *>(w + (sub + i * L) * 8 + 4);
+            }
+#pragma unroll
+        for (int i = 0; i < KEEP; ++i)
+            if (sub + i * L < chunks) square(raw[i], sub + i * L);
+    } else {
+#pragma unroll 4
+        for (int c = sub; c < chunks; c += L) square(ld16(xr + c * 8), c);
     }
     __syncthreads();
+    // the chain, 64 terms at a time
     float ss = 0.0f;
-    int d = 0;
-    for (; d + 64 <= D; d += 64) {
-        f32x4_t v[16];
+    const int blocks = D / 64;
+    f32x4_t v[AHEAD][16];
+    auto fetch = [&](int set, int blk) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = *reinterpret_cast<const f32x4_t *>(sr + d + i * 4);
+        for (int i = 0; i < 16; ++i) v[set][i] = *reinterpret_cast<const f32x4_t *>(sr + blk * 64 + i * 4);
+    };
+    auto add = [&](int set) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) ss = ss + v[i][0] + v[i][1] + v[i][2] + v[i][3];
+        for (int i = 0; i < 16; ++i) ss = ss + v[set][i][0] + v[set][i][1] + v[set][i][2] + v[set][i][3];
+    };
+    if constexpr (AHEAD == 2) {
+        if (blocks > 0) fetch(0, 0);
+        for (int b = 0; b + 1 < blocks; b += 2) {
+            fetch(1, b + 1);
+            add(0);
+            fetch(0, min(b + 2, blocks - 1));
+            add(1);
+        }
+        if (blocks & 1) add(0);
+    } else {
+        for (int b = 0; b < blocks; ++b) {
+            fetch(0, b);
+            add(0);
+        }
     }
-    for (; d < D; d += 8) {
-        const f32x4_t u = *reinterpret_cast<const f32x4_t *>(sr + d), v = *reinterpret_cast<const f32x4_t *>(sr + d + 4);
-        ss = ss + u[0] + u[1] + u[2] + u[3] + v[0] + v[1] + v[2] + v[3];
+    for (int d = blocks * 64; d < D; d += 8) {
+        const f32x4_t u = *reinterpret_cast<const f32x4_t *>(sr + d), t = *reinterpret_cast<const f32x4_t *>(sr + d + 4);
+        ss = ss + u[0] + u[1] + u[2] + u[3] + t[0] + t[1] + t[2] + t[3];
     }
     const float scale = 1.0f / sqrtf(ss / (float)D + eps);
     if (!valid) return;
-#pragma unroll 4
-    for (int c = sub; c < chunks; c += L) {
+    auto finish = [&](u32x4_t x8, f32x4_t g0, f32x4_t g1, int c) {
         float f[8];
-        unpack_bf16x8(ld16(xr + c * 8), f);
+        unpack_bf16x8(x8, f);
+        const float g[8] = {g0[0], g0[1], g0[2], g0[3], g1[0], g1[1], g1[2], g1[3]};
         u32x4_t o;
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
-            const float a = bf2f(f2bf(f[2 * h] * scale)) * w[c * 8 + 2 * h];
-            const float b = bf2f(f2bf(f[2 * h + 1] * scale)) * w[c * 8 + 2 * h + 1];
-            o[h] = pack_bf16x2(a, b);
-        }
+        for (int h = 0; h < 4; ++h)
+            o[h] = pack_bf16x2(bf2f(f2bf(f[2 * h] * scale)) * g[2 * h], bf2f(f2bf(f[2 * h + 1] * scale)) * g[2 * h + 1]);
         *reinterpret_cast<u32x4_t *>(out + r * D + c * 8) = o;
+    };
+    if (kept) {
+#pragma unroll
+        for (int i = 0; i < KEEP; ++i)
+            if (sub + i * L < chunks) finish(raw[i], gain[i][0], gain[i][1], sub + i * L);
+    } else {
+#pragma unroll 4
+        for (int c = sub; c < chunks; c += L)
+            finish(ld16(xr + c * 8), *reinterpret_cast<const f32x4_t *>(w + c * 8),
+                   *reinterpret_cast<const f32x4_t *>(w + c * 8 + 4), c);
     }
 }
 
