@@ -11,7 +11,11 @@
 // (x: [2^-63, 2^65), w: [2^-67, 2^61)), so that a product is below 2^126 and a multiple of 2^-144.  The check is an
 // add and an AND per pair of values (adding 64 or 68 to the exponent field sets its top bit exactly inside the
 // window); zeros fail it and are sorted out in a second look at the rows that were staged.  A tile that holds any
-// other value (infinities and NaN among them) is computed again with separate multiplies and adds.
+// other value (infinities and NaN among them) is computed again, the chunks of k that hold one with separate multiplies
+// and adds on the operands as they are laid out for the matrix instructions.  631 x 1024 x 3072: 47 us with none, 145
+// with one column of x outside, 647 with one value in every 16 of k; a plain multiply-add kernel takes 370 with any
+// input, so inputs that are outside throughout are slower here (32 x 151936 x 1024: 1121 us against 428) and rare ones
+// are faster (255 us).
 //
 // What bounds it.  f32 matrix instructions run at 155 TFLOP/s (1/16 of bf16) and share their issue slots with the
 // VALU: measured, every VALU instruction beside them adds its full 4 cycles.  So operands are widened to f32 once per
@@ -22,8 +26,8 @@
 //
 // Small steps (decode) are bound by the chain of one output instead: 8 cycles per k, 3.4 us at K = 1024.  There a
 // wave owns a single 16 x 16 tile and staging is left to producer waves of the same workgroup, which sit on the other
-// SIMDs, so the chain's SIMD does nothing else (K = 3072, N = 1024, 32 rows: 17.3 us; with the staging in the same wave
-// 26 us; one output per lane with 256-column workgroups, as multiplies and adds: 400 us).
+// SIMDs, so the chain's SIMD does nothing else (K = 3072, N = 1024, 32 rows: 16.3 us; with the staging in the same wave
+// 26 us; one output per lane with 256-column workgroups, as multiplies and adds: 343 us).
 #include "hip_common.h"
 
 #include <algorithm>
@@ -90,17 +94,8 @@ __device__ __forceinline__ void lin_put(const LinArgs &a, const LinOut &out, int
     else
         static_cast<bf16_t *>(out.y)[o] = __builtin_bit_cast(bf16_t, (__bf16)v);
 }
-// One output as the reference computes it: separate multiplies and adds.
-__device__ __forceinline__ float lin_plain(const bf16_t *xr, const bf16_t *wr, int K) {
-    float s = 0.0f;
-    for (int k = 0; k < K; k += 8) {
-        float xv[8], wv[8];
-        unpack_bf16x8(ld16(xr + k), xv);
-        unpack_bf16x8(ld16(wr + k), wv);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s = s + xv[e] * wv[e];
-    }
-    return s;
+__device__ __forceinline__ float lin_from_lane(float v, int lane) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(lane << 2, __builtin_bit_cast(int, v)));
 }
 
 // The order of one step's instructions: the LDS reads spread between the matrix instructions, then the staging's VALU
@@ -122,6 +117,11 @@ __device__ __forceinline__ void lin_interleave() {
         __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
     }
     __builtin_amdgcn_sched_group_barrier(0x008, PRODUCTS, 0);
+}
+
+template <class F, int... Is>
+__device__ __forceinline__ void lin_each(F f, std::integer_sequence<int, Is...>) {
+    (f(std::integral_constant<int, Is>{}), ...);
 }
 
 // A workgroup's tile: WM x WN waves of MT x NT blocks of 16 x 16 outputs, PW extra waves that only stage (0: every
@@ -162,8 +162,20 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
     bool is_w[T::SLOTS];
     u32x4_t raw[PF][T::SLOTS][2];
     int ahead = 0;  // next chunk to load
-    uint32_t bad = 0;
-    auto load = [&](u32x4_t (&r)[T::SLOTS][2]) {
+    bool bad = false;
+    auto begin = [&]() __attribute__((always_inline)) {
+        ahead = 0;
+#pragma unroll
+        for (int s = 0; s < T::SLOTS; ++s) {
+            const int i = sid + s * T::STAGERS, row = min(i / T::UNITS, T::ROWS - 1), u = i % T::UNITS;
+            is_w[s] = row < T::TN;
+            const long r = is_w[s] ? min(n0 + row, out.N - 1) : min(m0 + row - T::TN, a.M - 1);
+            koff[s] = u * 16;
+            src[s] = (is_w[s] ? out.w : a.x) + r * K + u * 16;
+            dst[s] = row * T::STRIDE + u * 16;
+        }
+    };
+    auto load = [&](u32x4_t (&r)[T::SLOTS][2]) __attribute__((always_inline)) {
 #pragma unroll
         for (int s = 0; s < T::SLOTS; ++s)
             if (T::has(sid, s))
@@ -184,7 +196,7 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
                 if (T::has(sid, s) && koff[s] + h * 8 < tail) r[s][h] = ld16(src[s] + base + h * 8);
             }
     };
-    auto stage_put = [&](const u32x4_t (&r)[T::SLOTS][2], int buf) {
+    auto stage_put = [&](const u32x4_t (&r)[T::SLOTS][2], int buf) __attribute__((always_inline)) {
         uint32_t in = LIN_IN;
 #pragma unroll
         for (int s = 0; s < T::SLOTS; ++s) {
@@ -203,7 +215,7 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
         }
         return in;
     };
-    auto stage_check = [&](const u32x4_t (&r)[T::SLOTS][2], uint32_t in) {
+    auto stage_check = [&](const u32x4_t (&r)[T::SLOTS][2], uint32_t in) __attribute__((always_inline)) {
         if (__builtin_expect(__ballot(in != LIN_IN) != 0, 0)) {
 #pragma unroll
             for (int s = 0; s < T::SLOTS; ++s) {
@@ -224,8 +236,14 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
     const int frag = (lane & 15) * T::STRIDE + (lane >> 4) * 4;
     const int wbase = wn * NT * 16 * T::STRIDE + frag, xbase = (T::TN + wm * MT * 16) * T::STRIDE + frag;
     f32x4_t acc[MT][NT];
+    auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    };
     f32x4_t wf[2][T::UNITS][NT], xf[2][T::UNITS][MT];
-    auto fetch = [&](int set) {
+    auto fetch = [&](int set) __attribute__((always_inline)) {
         const float *b = lds[set];
 #pragma unroll
         for (int s = 0; s < T::UNITS; ++s) {
@@ -237,7 +255,7 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
                 xf[set][s][m] = *reinterpret_cast<const f32x4_t *>(b + xbase + m * 16 * T::STRIDE + s * 16);
         }
     };
-    auto compute = [&](int set) {
+    auto compute = [&](int set) __attribute__((always_inline)) {
 #pragma unroll
         for (int s = 0; s < T::UNITS; ++s)
 #pragma unroll
@@ -250,21 +268,37 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
                             __builtin_amdgcn_mfma_f32_16x16x4f32(wf[set][s][n][j], xf[set][s][m][j], acc[m][n], 0, 0, 0);
     };
 
+    // The same operands with separate multiplies and adds, as the reference does: each k in turn reaches the lanes of
+    // its outputs by lane exchanges.  k = 16 s + 4 j + q of the chunk, q ascending.
+    auto separate4 = [&](int set, auto at) __attribute__((always_inline)) {
+        constexpr int s = decltype(at)::value / 4;
+        constexpr int j = decltype(at)::value % 4;
+#pragma unroll 1
+        for (int q = 0; q < 4; ++q) {
+            float xv[MT];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) xv[m] = lin_from_lane(xf[set][s][m][j], q * 16 + (lane & 15));
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float wv = lin_from_lane(wf[set][s][n][j], q * 16 + (lane >> 4) * 4 + r);
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) acc[m][n][r] = acc[m][n][r] + xv[m] * wv;
+                }
+        }
+    };
+    auto separate = [&](int set) __attribute__((always_inline)) {
+        lin_each([&](auto at) __attribute__((always_inline)) { separate4(set, at); },
+                 std::make_integer_sequence<int, T::UNITS * 4>{});
+    };
     // Step i: the products of chunk i, the fragments of chunk i + 1, the staging of chunk i + 2, the loads of chunk
     // i + 2 + PF.
     auto run = [&](auto stager, auto multiplier) {
         constexpr bool S = decltype(stager)::value, C = decltype(multiplier)::value;
         const int chunks = full + (tail > 0);
         if constexpr (S) {
-#pragma unroll
-            for (int s = 0; s < T::SLOTS; ++s) {
-                const int i = sid + s * T::STAGERS, row = min(i / T::UNITS, T::ROWS - 1), u = i % T::UNITS;
-                is_w[s] = row < T::TN;
-                const long r = is_w[s] ? min(n0 + row, out.N - 1) : min(m0 + row - T::TN, a.M - 1);
-                koff[s] = u * 16;
-                src[s] = (is_w[s] ? out.w : a.x) + r * K + u * 16;
-                dst[s] = row * T::STRIDE + u * 16;
-            }
+            begin();
             if (full > 0) {
 #pragma unroll
                 for (int p = 0; p < PF; ++p) load(raw[p]);
@@ -273,12 +307,7 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
             stage(raw[0], 0);
             if (full > 0) load(raw[0]);
         }
-        if constexpr (C) {
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-#pragma unroll
-                for (int n = 0; n < NT; ++n) acc[m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        }
+        if constexpr (C) clear();
         __syncthreads();
         if constexpr (C) fetch(0);
         if constexpr (S) {
@@ -332,14 +361,37 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
         else
             run(std::true_type{}, std::false_type{});
     }
-    if (__builtin_expect(__syncthreads_or((int)bad), 0)) {  // a value outside its window
-        for (int i = tid; i < T::TM * T::TN; i += T::THREADS) {
-            const int m = m0 + i / T::TN, n = n0 + i % T::TN;
-            if (m < a.M && n < out.N) lin_put(a, out, m, n, lin_plain(a.x + (long)m * K, out.w + (long)n * K, K));
+    const bool stager = !PW || wave >= T::WAVES, multiplier = !PW || wave < T::WAVES;
+    if (__builtin_expect(__syncthreads_or((int)bad), 0)) {  // a value outside its window: the tile again
+        auto next = [&](int c) {
+            if (c < full)
+                load(raw[0]);
+            else if (c * KC < K)
+                load_tail(raw[0]);
+        };
+        clear();
+        if (stager) {
+            begin();
+            next(0);
         }
-        return;
+        for (int c = 0; c * KC < K; ++c) {
+            bad = false;
+            if (stager) {
+                stage_check(raw[0], stage_put(raw[0], 0));
+                next(c + 1);
+            }
+            const bool apart = __syncthreads_or((int)bad);
+            if (multiplier) {
+                fetch(0);
+                if (apart)
+                    separate(0);
+                else
+                    compute(0);
+            }
+            __syncthreads();
+        }
     }
-    if (PW && wave >= T::WAVES) return;
+    if (!multiplier) return;
     // D of the instruction: its columns are rows of x, a lane's four values are consecutive columns of y
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
@@ -420,11 +472,11 @@ __global__ void __launch_bounds__(256) linear_stream_kernel(const LinArgs a) {
         xr[set] = u32x4_t{0u, 0u, 0u, 0u};
         if (xpiece * 8 < tail) xr[set] = ld16(xp + o);
     };
-    uint32_t bad = 0;
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
     auto use = [&](int set) {
         float wf[4][8], xf[8];
         uint32_t in = LIN_IN;
+        bool bad = false;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             unpack_bf16x8(wr[set][i], wf[i]);
@@ -443,6 +495,20 @@ __global__ void __launch_bounds__(256) linear_stream_kernel(const LinArgs a) {
                              lin_half_ok(wr[set][i][d] >> 16, LIN_W_BIAS));
                 bad |= !(lin_half_ok(xr[set][d] & 0xffffu, LIN_X_BIAS) && lin_half_ok(xr[set][d] >> 16, LIN_X_BIAS));
             }
+        }
+        if (__builtin_expect(__ballot(bad) != 0, 0)) {  // a value outside its window: separate multiplies and adds
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll 1
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float wv = lin_from_lane(wf[i][e], h * 32 + (lane & 31));
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            acc[r] = acc[r] + lin_from_lane(xf[e], half * 32 + (2 * i + h) * 4 + r) * wv;
+                    }
+            return;
         }
         // the VALU work stays in one piece: each change between it and the matrix cores costs 8 cycles
         __builtin_amdgcn_sched_barrier(0);
@@ -464,13 +530,6 @@ __global__ void __launch_bounds__(256) linear_stream_kernel(const LinArgs a) {
     for (int p = 0; p < PF; ++p) {
         if (c + p == full && tail) load_tail(p);
         if (c + p < full + (tail > 0)) use(p);
-    }
-    if (__builtin_expect(__syncthreads_or((int)bad), 0)) {  // a value outside its window
-        for (int i = threadIdx.x; i < a.M * STREAM_COLS; i += 256) {
-            const int m = i / STREAM_COLS, n = b0 + i % STREAM_COLS;
-            if (n < out.N) lin_put(a, out, m, n, lin_plain(a.x + (long)m * K, out.w + (long)n * K, K));
-        }
-        return;
     }
     const int n = n0 + (lane & 31);
     if (n >= out.N) return;

@@ -60,7 +60,8 @@ def test_linear_any_output_alignment(gpu, N, offset, y_f32):
     check(draw(rng, 19, 48), draw(rng, N, 48), y_f32, offset)
 
 
-@pytest.mark.parametrize("M,N,K", [(9, 70, 136), (40, 2000, 72), (12, 8300, 72), (7, 8300, 136), (200, 1100, 200), (512, 2048, 40)])
+@pytest.mark.parametrize("M,N,K", [(9, 70, 136), (40, 2000, 72), (12, 8300, 72), (7, 8300, 136), (200, 1100, 200), (512, 2048, 40),
+                                   (200, 3001, 104), (1000, 3060, 40), (2048, 6144, 16)])
 @pytest.mark.parametrize("what", ["zeros", "tiny", "huge", "nonfinite", "edges"])
 def test_linear_values_outside_the_exact_window(gpu, M, N, K, what):
     """Zeros stay on the fast path; values whose products leave f32's exact range (or are not finite) must take the
