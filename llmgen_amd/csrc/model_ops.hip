@@ -1,12 +1,11 @@
 // model_ops.hip -- the non-attention ops of the Qwen3 forward except linear (embedding, RMSNorm, NEOX RoPE, SiLU,
-// add, mul, gather_last, sampling) for the end-to-end greedy-token check, and the fused q/k norm + RoPE + KV
-// write that replaces five of them before attention.
+// add, mul, gather_last, sampling), and the fused q/k norm + RoPE + KV write that replaces five of them before
+// attention.
 //
-// These kernels trade speed for reproducibility: every output is computed in the order the reference CPU
+// Order and roundings come first, speed within them: every output is computed in the order the reference CPU
 // backend uses (src/backend/cpu/*.zig), with one IEEE rounding per f32 multiply / add / divide / sqrt and one
 // RNE rounding to bf16 per stored value, so a forward built from them matches the CPU backend bit for bit
-// outside attention.  Contraction into FMAs is switched off for the whole file for that reason.  They are not
-// part of the measured hot path.
+// outside attention.  Contraction into FMAs is switched off for the whole file for that reason.
 #include "hip_common.h"
 
 #include <math.h>
