@@ -11,11 +11,11 @@
 // (x: [2^-63, 2^65), w: [2^-67, 2^61)), so that a product is below 2^126 and a multiple of 2^-144.  The check is an
 // add and an AND per pair of values (adding 64 or 68 to the exponent field sets its top bit exactly inside the
 // window); zeros fail it and are sorted out in a second look at the rows that were staged.  A tile that holds any
-// other value (infinities and NaN among them) is computed again, the chunks of k that hold one with separate multiplies
-// and adds on the operands as they are laid out for the matrix instructions.  631 x 1024 x 3072: 47 us with none, 145
-// with one column of x outside, 647 with one value in every 16 of k; a plain multiply-add kernel takes 370 with any
-// input, so inputs that are outside throughout are slower here (32 x 151936 x 1024: 1121 us against 428) and rare ones
-// are faster (255 us).
+// other value (infinities and NaN among them) is computed again with the products of the chunks that hold one rounded
+// before they are added.  If one of the first two chunks holds one, the first pass ends there.  631 x 1024 x 3072: 46 us
+// with none, 86 with one column of x outside, 190 with one value in every 16 of k (the plain multiply-add kernel that
+// these replace: 368 with any input); 2048 x 6144 x 2048: 371, 502 and 1084 us (1704); 32 x 151936 x 1024: 96, 136 and
+// 241 us (431).
 //
 // What bounds it.  f32 matrix instructions run at 155 TFLOP/s (1/16 of bf16) and share their issue slots with the
 // VALU: measured, every VALU instruction beside them adds its full 4 cycles.  So operands are widened to f32 once per
@@ -94,9 +94,6 @@ __device__ __forceinline__ void lin_put(const LinArgs &a, const LinOut &out, int
     else
         static_cast<bf16_t *>(out.y)[o] = __builtin_bit_cast(bf16_t, (__bf16)v);
 }
-__device__ __forceinline__ float lin_from_lane(float v, int lane) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(lane << 2, __builtin_bit_cast(int, v)));
-}
 
 // The order of one step's instructions: the LDS reads spread between the matrix instructions, then the staging's VALU
 // work in one piece, then its LDS writes spread likewise.  A wave issues in order and its LDS queue is short, so reads
@@ -119,11 +116,6 @@ __device__ __forceinline__ void lin_interleave() {
     __builtin_amdgcn_sched_group_barrier(0x008, PRODUCTS, 0);
 }
 
-template <class F, int... Is>
-__device__ __forceinline__ void lin_each(F f, std::integer_sequence<int, Is...>) {
-    (f(std::integral_constant<int, Is>{}), ...);
-}
-
 // A workgroup's tile: WM x WN waves of MT x NT blocks of 16 x 16 outputs, PW extra waves that only stage (0: every
 // wave stages), KC values of k per LDS chunk.
 template <int MT, int NT, int WM, int WN, int PW, int KC>
@@ -133,19 +125,23 @@ struct LinTile {
     static constexpr int UNITS = KC / 16;  // 16 consecutive k of a row: one staging slot
     static constexpr int WORK = ROWS * UNITS, SLOTS = (WORK + STAGERS - 1) / STAGERS;
     static constexpr int STRIDE = KC + 4;  // f32 per staged row
-    static constexpr int LDS = 2 * ROWS * STRIDE * 4;
     // whether slot s of a staging thread has work (whole waves drop out of the last slot)
     static __device__ __forceinline__ bool has(int id, int s) {
         return (s + 1) * STAGERS <= WORK || id + s * STAGERS < WORK;
     }
 };
 
+// "At least two waves a SIMD" keeps the sums in ordinary registers, where the VALU adds to them without moves.  Not so in
+// the kernels with producer waves, which are 2 % faster without it (32 x 1024 x 3072: 15.9 and 16.3 us; with values outside
+// the window throughout 83 and 58 us).
 template <int MT, int NT, int WM, int WN, int PW, int KC, int PF>
-__global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinArgs a) {
+__global__ void __launch_bounds__((WM * WN + PW) * 64, PW ? 1 : 2) linear_kernel(const LinArgs a) {
     using T = LinTile<MT, NT, WM, WN, PW, KC>;
     static_assert(PF % 2 == 0, "chunk parity names the LDS buffer");
     __shared__ __attribute__((aligned(16))) float lds[2][T::ROWS * T::STRIDE];
+    __shared__ int flag[3];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid == 0) flag[0] = 0;
     // tiles in order of columns, each XCD (block index mod 8) a contiguous range of them
     const int tiles = gridDim.x;
     const int per = tiles >> 3, rem = tiles & 7, xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
@@ -268,35 +264,53 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
                             __builtin_amdgcn_mfma_f32_16x16x4f32(wf[set][s][n][j], xf[set][s][m][j], acc[m][n], 0, 0, 0);
     };
 
-    // The same operands with separate multiplies and adds, as the reference does: each k in turn reaches the lanes of
-    // its outputs by lane exchanges.  k = 16 s + 4 j + q of the chunk, q ascending.
-    auto separate4 = [&](int set, auto at) __attribute__((always_inline)) {
-        constexpr int s = decltype(at)::value / 4;
-        constexpr int j = decltype(at)::value % 4;
+    // The first `units` units of a staged chunk; `apart`: with separate multiplies and adds, as the reference does.
+    // v_mfma_f32_16x16x1 takes the same operands and gives the products of its four k apart, each fma(x, w, +0) and so
+    // rounded once; the VALU adds them k by k.  (A product of -0 may come out as +0, but no sum is ever -0, so that does
+    // not show.)  96 cycles for 16 x 16 x 4 products on one SIMD, against 32 fused and 128 as VALU multiplies and adds.
+    auto products = [&](const float *b, int units, bool apart) __attribute__((always_inline)) {
 #pragma unroll 1
-        for (int q = 0; q < 4; ++q) {
-            float xv[MT];
-#pragma unroll
-            for (int m = 0; m < MT; ++m) xv[m] = lin_from_lane(xf[set][s][m][j], q * 16 + (lane & 15));
+        for (int s = 0; s < units; ++s) {
+            f32x4_t w4[NT], x4[MT];
 #pragma unroll
             for (int n = 0; n < NT; ++n)
+                w4[n] = *reinterpret_cast<const f32x4_t *>(b + wbase + n * 16 * T::STRIDE + s * 16);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float wv = lin_from_lane(wf[set][s][n][j], q * 16 + (lane >> 4) * 4 + r);
+            for (int m = 0; m < MT; ++m)
+                x4[m] = *reinterpret_cast<const f32x4_t *>(b + xbase + m * 16 * T::STRIDE + s * 16);
+            if (apart) {
+                f32x16_t p[2];  // one block's products form while the other's are added
+                constexpr int ALL = 4 * MT * NT;
 #pragma unroll
-                    for (int m = 0; m < MT; ++m) acc[m][n][r] = acc[m][n][r] + xv[m] * wv;
+                for (int t = 0; t <= ALL; ++t) {
+                    if (t < ALL)
+                        p[t & 1] = __builtin_amdgcn_mfma_f32_16x16x1f32(w4[t % NT][t / (MT * NT)],
+                                                                        x4[t / NT % MT][t / (MT * NT)], f32x16_t{}, 0, 0, 0);
+                    if (t > 0) {
+                        f32x4_t &sum = acc[(t - 1) / NT % MT][(t - 1) % NT];
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) sum[i & 3] = sum[i & 3] + p[(t - 1) & 1][i];
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int m = 0; m < MT; ++m)
+#pragma unroll
+                        for (int n = 0; n < NT; ++n)
+                            acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(w4[n][j], x4[m][j], acc[m][n], 0, 0, 0);
+            }
         }
     };
-    auto separate = [&](int set) __attribute__((always_inline)) {
-        lin_each([&](auto at) __attribute__((always_inline)) { separate4(set, at); },
-                 std::make_integer_sequence<int, T::UNITS * 4>{});
-    };
     // Step i: the products of chunk i, the fragments of chunk i + 1, the staging of chunk i + 2, the loads of chunk
-    // i + 2 + PF.
+    // i + 2 + PF.  Returns whether a value lies outside its window (then the sums are of no use): asked after the first
+    // two chunks and at the end.
+    const int chunks = full + (tail > 0);
+    auto flagged = [&](int i) { return __builtin_amdgcn_readfirstlane(flag[i]) != 0; };
     auto run = [&](auto stager, auto multiplier) {
         constexpr bool S = decltype(stager)::value, C = decltype(multiplier)::value;
-        const int chunks = full + (tail > 0);
         if constexpr (S) {
             begin();
             if (full > 0) {
@@ -314,8 +328,10 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
             if (full == 1 && tail) load_tail(raw[1]);
             if (chunks > 1) stage(raw[1], 1);
             if (full > 0) load(raw[1]);
+            if (bad) flag[0] = 1;
         }
         __syncthreads();
+        if (__builtin_expect(flagged(0), 0)) return true;
         int i = 0;
         for (; i + PF + 2 <= full; i += PF) {
 #pragma unroll
@@ -350,45 +366,57 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64) linear_kernel(const LinAr
                 if constexpr (S)
                     if (i + p + 2 < chunks) stage(raw[(p + 2) % PF], p & 1);
                 if constexpr (C) compute(p & 1);
+                if constexpr (S)
+                    if (bad) flag[0] = 1;
                 __syncthreads();
             }
+        return flagged(0);
     };
+    const bool multiplier = !PW || __builtin_amdgcn_readfirstlane(wave) < T::WAVES, stager = !PW || !multiplier;
+    bool again;
     if constexpr (PW == 0) {
-        run(std::true_type{}, std::true_type{});
+        again = run(std::true_type{}, std::true_type{});
     } else {
-        if (__builtin_amdgcn_readfirstlane(wave) < T::WAVES)
-            run(std::false_type{}, std::true_type{});
+        if (multiplier)
+            again = run(std::false_type{}, std::true_type{});
         else
-            run(std::true_type{}, std::false_type{});
+            again = run(std::true_type{}, std::false_type{});
     }
-    const bool stager = !PW || wave >= T::WAVES, multiplier = !PW || wave < T::WAVES;
-    if (__builtin_expect(__syncthreads_or((int)bad), 0)) {  // a value outside its window: the tile again
-        auto next = [&](int c) {
-            if (c < full)
-                load(raw[0]);
-            else if (c * KC < K)
-                load_tail(raw[0]);
-        };
+    if (__builtin_expect(again, 0)) {  // a value outside its window: the tile again, chunks that hold one apart
         clear();
-        if (stager) {
-            begin();
-            next(0);
-        }
-        for (int c = 0; c * KC < K; ++c) {
-            bad = false;
-            if (stager) {
-                stage_check(raw[0], stage_put(raw[0], 0));
+        if (chunks <= 2) {  // they are both in LDS still
+            if (multiplier)
+                for (int c = 0; c < chunks; ++c) products(lds[c], c < full ? T::UNITS : (tail + 15) / 16, true);
+        } else {
+            // Step c: the products of chunk c, the staging of chunk c + 1, the load of chunk c + 2; flag[c % 3]: chunk c
+            // is to be kept apart.
+            auto next = [&](int c) {
+                if (c < full)
+                    load(raw[0]);
+                else if (c < chunks)
+                    load_tail(raw[0]);
+            };
+            auto put = [&](int c) {
+                bad = false;
+                stage(raw[0], c & 1);
+                if (bad) flag[c % 3] = 1;
                 next(c + 1);
-            }
-            const bool apart = __syncthreads_or((int)bad);
-            if (multiplier) {
-                fetch(0);
-                if (apart)
-                    separate(0);
-                else
-                    compute(0);
+            };
+            if (stager) {
+                begin();
+                next(0);
             }
             __syncthreads();
+            if (tid < 3) flag[tid] = 0;
+            __syncthreads();
+            if (stager) put(0);
+            __syncthreads();
+            for (int c = 0; c < chunks; ++c) {
+                if (stager && c + 1 < chunks) put(c + 1);
+                if (multiplier) products(lds[c & 1], c < full ? T::UNITS : (tail + 15) / 16, flagged(c % 3));
+                if (tid == 0) flag[(c + 2) % 3] = 0;
+                __syncthreads();
+            }
         }
     }
     if (!multiplier) return;
@@ -446,7 +474,26 @@ __device__ __forceinline__ f32x4_t stream_products(f32x4_t acc, const float (&wf
     return acc;
 }
 
-__global__ void __launch_bounds__(256) linear_stream_kernel(const LinArgs a) {
+// The same with the products rounded before they are added, four k at a time (see `products` above).
+template <int... Qs>
+__device__ __forceinline__ f32x4_t stream_apart(f32x4_t acc, const float (&wf)[4][8], const float (&xf)[8],
+                                                std::integer_sequence<int, Qs...>) {
+    auto four = [&](auto q) __attribute__((always_inline)) {
+        constexpr int K0 = decltype(q)::value * 4;
+        const f32x4_t p[4] = {stream_products(f32x4_t{}, wf, xf, std::integer_sequence<int, K0>{}),
+                              stream_products(f32x4_t{}, wf, xf, std::integer_sequence<int, K0 + 1>{}),
+                              stream_products(f32x4_t{}, wf, xf, std::integer_sequence<int, K0 + 2>{}),
+                              stream_products(f32x4_t{}, wf, xf, std::integer_sequence<int, K0 + 3>{})};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[r] = acc[r] + p[i][r];
+    };
+    (four(std::integral_constant<int, Qs>{}), ...);
+    return acc;
+}
+
+__global__ void __launch_bounds__(256, 2) linear_stream_kernel(const LinArgs a) {
     constexpr int KC = STREAM_KC, PF = STREAM_PF;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int b0;
@@ -496,18 +543,8 @@ __global__ void __launch_bounds__(256) linear_stream_kernel(const LinArgs a) {
                 bad |= !(lin_half_ok(xr[set][d] & 0xffffu, LIN_X_BIAS) && lin_half_ok(xr[set][d] >> 16, LIN_X_BIAS));
             }
         }
-        if (__builtin_expect(__ballot(bad) != 0, 0)) {  // a value outside its window: separate multiplies and adds
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll 1
-                for (int h = 0; h < 2; ++h)
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const float wv = lin_from_lane(wf[i][e], h * 32 + (lane & 31));
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            acc[r] = acc[r] + lin_from_lane(xf[e], half * 32 + (2 * i + h) * 4 + r) * wv;
-                    }
+        if (__builtin_expect(__ballot(bad) != 0, 0)) {  // a value outside its window: products and sums apart
+            acc = stream_apart(acc, wf, xf, std::make_integer_sequence<int, KC / 4>{});
             return;
         }
         // the VALU work stays in one piece: each change between it and the matrix cores costs 8 cycles

@@ -121,3 +121,42 @@ def test_linear_add_equals_linear_then_add(gpu, M, N, what):
     assert lib().hip_last_error() == 0
     got = yd.cpu().numpy()[:M * N].view(np.uint16).reshape(M, N)
     np.testing.assert_array_equal(got, O.add(res.reshape(-1), O.linear(x, w).reshape(-1)).reshape(M, N))
+
+
+# Per kernel of the dispatch (at 256 CUs) a K of at least two trips of its pipelined loop and a remainder: (M, N, K) and the
+# chunk of k, whole chunks
+LOOPS = [(17, 900, 968, 128),    # one block a workgroup: 7
+         (40, 2000, 712, 64),    # two blocks, loop of four chunks: 11
+         (5, 8200, 712, 64),     # stream, loop of three stages: 11
+         (12, 8300, 424, 64),    # 9 to 16 rows: 6
+         (17, 4104, 424, 64),    # 32 x 32: 6
+         (65, 5482, 248, 32),    # 32 x 96: 7
+         (97, 6171, 248, 32),    # 64 x 64: 7
+         (353, 6171, 200, 32),   # 64 x 192: 6
+         (517, 5800, 248, 32)]   # 128 x 128: 7
+
+
+@pytest.mark.parametrize("M,N,K,chunk", LOOPS)
+@pytest.mark.parametrize("operand", ["x", "w"])
+@pytest.mark.parametrize("what", ["tiny", "huge"])
+def test_linear_one_chunk_outside_the_exact_window(gpu, M, N, K, chunk, operand, what):
+    """One output of the last tile is the sum of two products from one chunk of k, all its other terms are zeros, and
+    fused additions would give another sum: 2^-149 + 2^-150 (2^-149 as separate operations, 2^-148 fused), or
+    -1.5 * 2^127 + 2^128 (+inf, 2^126 fused).  The chunk is the first, one in the middle, the last whole one, the
+    remainder."""
+    far, near = {"tiny": ((2.0**-90, 2.0**-90), (2.0**-59, 2.0**-60)),
+                 "huge": ((-1.5 * 2.0**100, 2.0**100), (2.0**27, 2.0**28))}[what]
+    rng = np.random.default_rng(M + N)
+    whole = K // chunk
+    x0, w0 = draw(rng, M, K), draw(rng, N, K, std=0.05)
+    clean = O.linear(x0, w0, out_bf16=False)
+    for at in (0, whole // 2, whole - 1, whole):
+        x, w, k = x0.copy(), w0.copy(), at * chunk + 3
+        row, col = (x, w) if operand == "x" else (w, x)
+        row[-1], col[-1, k:k + 2] = 0, O.f32_to_bf16(np.array(near, np.float32))
+        row[-1, k:k + 2] = O.f32_to_bf16(np.array(far, np.float32))
+        ref = clean.copy()  # the special row and column anew, the rest is as it was
+        ref[-1:], ref[:, -1:] = O.linear(x[-1:], w, out_bf16=False), O.linear(x, w[-1:], out_bf16=False)
+        assert ref[-1, -1] == (np.float32(2.0**-149) if what == "tiny" else np.inf)
+        got = run(x, w, y_f32=True)
+        np.testing.assert_array_equal(got.view(np.uint32), ref.view(np.uint32))
