@@ -137,6 +137,12 @@ LOOPS = [(17, 900, 968, 128),    # one block a workgroup: 7
 
 
 @pytest.mark.parametrize("M,N,K,chunk", LOOPS)
+def test_linear_main_loops_bit_exact(gpu, M, N, K, chunk):
+    rng = np.random.default_rng(M + N + K)
+    check(draw(rng, M, K), draw(rng, N, K, std=0.05), y_f32=M % 2 == 1)
+
+
+@pytest.mark.parametrize("M,N,K,chunk", LOOPS)
 @pytest.mark.parametrize("operand", ["x", "w"])
 @pytest.mark.parametrize("what", ["tiny", "huge"])
 def test_linear_one_chunk_outside_the_exact_window(gpu, M, N, K, chunk, operand, what):
@@ -160,3 +166,23 @@ def test_linear_one_chunk_outside_the_exact_window(gpu, M, N, K, chunk, operand,
         assert ref[-1, -1] == (np.float32(2.0**-149) if what == "tiny" else np.inf)
         got = run(x, w, y_f32=True)
         np.testing.assert_array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
+# the products' column tiles in the streaming, 9..16-row, 32 x 96, 64 x 64, 64 x 192 and 128 x 128 kernels, main loops included
+@pytest.mark.parametrize("M,Ns", [(1, (6144, 6144, 0)), (8, (5000, 3001, 1030)), (9, (6144, 6144, 0)),
+                                  (16, (5000, 3001, 1030)), (300, (6144, 6144, 0)), (700, (5000, 3001, 1030)),
+                                  (300, (5000, 3001, 1030)), (600, (6144, 6151, 0))])
+def test_linear3_wide_equals_single_products(gpu, M, Ns):
+    K, rng = 456, np.random.default_rng(M + sum(Ns))
+    x, ws = draw(rng, M, K), [draw(rng, max(n, 1), K, std=0.1) for n in Ns]
+    ws[1][0, 200] = 0x0001  # only tiles of the second product hold a value outside the window
+    xd, wd = torch.from_numpy(x.view(np.int16)).cuda(), [torch.from_numpy(w.view(np.int16)).cuda() for w in ws]
+    ys = [torch.full((M * n + 8,), 77, dtype=torch.int16, device="cuda") for n in Ns]
+    args = [a for y, w, n in zip(ys, wd, Ns) for a in ((y.data_ptr(), w.data_ptr(), n) if n else (None, None, 0))]
+    lib().hip_linear3(*args, xd.data_ptr(), M, K)
+    torch.cuda.synchronize()
+    assert lib().hip_last_error() == 0
+    for y, w, n in zip(ys, ws, Ns):
+        got, ref = y.cpu().numpy(), run(x, w, False)[:, :n] if n else np.zeros((M, 0), np.uint16)
+        assert (got[M * n:] == 77).all()
+        np.testing.assert_array_equal(got[:M * n].view(np.uint16).reshape(M, n), ref)
