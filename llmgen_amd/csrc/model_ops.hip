@@ -349,6 +349,19 @@ bool reject(const char *what) {
 
 unsigned blocks_for(size_t n, unsigned per) { return (unsigned)((n + per - 1) / per); }
 
+// Whether p is memory of the current device, where a compare-and-swap needs nothing from the bus (host memory: PCIe
+// atomics, which not every machine routes).  A query only, allowed while a stream is captured.
+bool on_this_device(const void *p) {
+    const hipError_t before = hipPeekAtLastError();
+    int dev = 0;
+    hipPointerAttribute_t at{};
+    if (hipGetDevice(&dev) == hipSuccess && hipPointerGetAttributes(&at, p) == hipSuccess)
+        return at.type == hipMemoryTypeDevice && at.device == dev;
+    (void)hipGetLastError();  // this query's own error; an earlier one stays known
+    if (before != hipSuccess) llmgen_record_error(before);
+    return false;
+}
+
 template <class Op>
 void elementwise(bf16_t *out, const bf16_t *a, const bf16_t *b, size_t n, Op op) {
     if (n == 0) return;
@@ -440,7 +453,8 @@ void hip_sample(int32_t *out_ids, const uint16_t *logits, const float *temps, co
         return;
     }
     // slices: enough workgroups to fill the chip eight times over (rows with noise take far longer than greedy ones)
-    const int slices = std::max(1, std::min(V / SLICE_MIN, 8 * llmgen_num_cus() / S));
+    int slices = std::max(1, std::min(V / SLICE_MIN, 8 * llmgen_num_cus() / S));
+    if (slices > 1 && !on_this_device(out_ids)) slices = 1;  // one workgroup a row, which writes its id with a plain store
     if (slices > 1) sample_start_kernel<<<blocks_for(S, 256), 256, 0, g_llmgen_stream>>>(out_ids, S);
     sample_rows_kernel<<<(unsigned)S * slices, ROW_THREADS, 0, g_llmgen_stream>>>(out_ids, logits, temps, seed, V,
                                                                                    slices);

@@ -98,3 +98,64 @@ def test_sample_slices(gpu, S, V):
             lib().hip_sample(out.data_ptr(), ld.data_ptr(), tdev.data_ptr(), seed.data_ptr(), S, V, None)
             torch.cuda.synchronize()
             np.testing.assert_array_equal(out.cpu().numpy(), O.sample(lg, t, seed=1234567))
+
+
+def test_sample_into_pinned_host_memory(gpu):
+    """Ids written straight to the host: no device-side read-modify-write of that memory (it would need PCIe atomics)."""
+    S, V = 3, 60007
+    rng = np.random.default_rng(8)
+    lg, temps = draw(rng, S, V), np.array([0.0, 0.8, 1.3], np.float32)
+    seed = torch.tensor([99], dtype=torch.int64, device="cuda")
+    ld, td = up(lg), up(temps)
+    out = torch.full((S,), -5, dtype=torch.int32, pin_memory=True)
+    lib().hip_sample(out.data_ptr(), ld.data_ptr(), td.data_ptr(), seed.data_ptr(), S, V, None)
+    torch.cuda.synchronize()
+    assert lib().hip_last_error() == 0
+    np.testing.assert_array_equal(out.numpy(), O.sample(lg, temps, seed=99))
+
+
+def test_mlp_and_sampling_captured(gpu):
+    """The products, norms and sampling of a step recorded into a graph: replayed on new inputs, with eager work in
+    between, each replay equals the eager launches."""
+    T, D, F, V = 20, 256, 520, 40960
+    L, rng = lib(), np.random.default_rng(4)
+    g = up((1 + 0.1 * rng.standard_normal(D)).astype(np.float32))
+    wg, wu, wd, wh = (up(draw(rng, n, k, std=0.05)) for n, k in ((F, D), (F, D), (D, F), (V, D)))
+    temps, seed = up(np.where(np.arange(T) % 3 == 1, 0.8, 0).astype(np.float32)), torch.tensor([7], device="cuda")
+    x, xn, gate, upp = (torch.zeros(T * n, dtype=torch.int16, device="cuda") for n in (D, D, F, F))
+    logits = torch.zeros(T * V, dtype=torch.int16, device="cuda")
+    ids = torch.zeros(T, dtype=torch.int32, device="cuda")
+
+    def step():
+        p = torch.Tensor.data_ptr
+        L.hip_rmsnorm(p(xn), p(x), p(g), T, D, 1e-6)
+        L.hip_linear3(p(gate), p(wg), F, p(upp), p(wu), F, None, None, 0, p(xn), T, D)
+        L.hip_silu_mul(p(gate), p(gate), p(upp), T * F)
+        L.hip_linear_add(p(x), p(x), p(gate), p(wd), T, D, F)
+        L.hip_linear(p(logits), 0, p(x), p(wh), T, V, D)
+        L.hip_sample(p(ids), p(logits), p(temps), p(seed), T, V, None)
+
+    inputs = [up(draw(rng, T * D)) for _ in range(4)]
+    refs = []
+    for v in inputs:
+        x.copy_(v)
+        step()
+        torch.cuda.synchronize()
+        refs.append((x.clone(), logits.clone(), ids.clone()))
+    assert L.hip_graph_begin() == 0
+    step()
+    graph = L.hip_graph_end()
+    assert graph, "capture failed"
+    try:
+        for v, ref in zip(inputs, refs):
+            x.copy_(v)
+            logits.zero_()
+            ids.fill_(-1)
+            torch.cuda.synchronize()
+            L.hip_graph_launch(graph)
+            torch.cuda.synchronize()
+            assert L.hip_last_error() == 0
+            for got, want in zip((x, logits, ids), ref):
+                assert torch.equal(got, want)
+    finally:
+        L.hip_graph_destroy(graph)
