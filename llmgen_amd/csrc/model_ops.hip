@@ -206,19 +206,14 @@ __global__ void gather_rows_kernel(bf16_t *out, const bf16_t *x, const int *idx,
 // What bit parity with the CPU backend fixes is kept as it is: the splitmix64 stream per (seed, row, index), the
 // uniform from its top 24 bits and the Gumbel value v / t - log(-log u), each f32 operation rounded once.
 //
-// A row is cut into slices, one workgroup each: a 151936-wide row is 2374 waves' worth of work, and drawing its noise
-// (two logarithms and two 64-bit products per value) takes one CU 70 us.  Slices of one row meet in out[row] itself:
-// it holds the index of the best candidate so far, whose key any workgroup can form again from the logits, so a
-// workgroup that found a better one replaces it with a compare-and-swap (retried while others do the same; every retry
-// means the row got better).  No scratch, and the result does not depend on the order: the largest key wins.
-// Measured, 32 rows of 151936: greedy 17.2 -> 10.1 us, a third of them with noise 69.7 -> 17.6 us (one workgroup per row).
-constexpr int ROW_THREADS = 256;
-// Values of a slice at least: with noise 32 per lane; greedy rows, whose scan is a plain read, use the first
-// 1 / GREEDY_SLICES of the slices, since the compare-and-swaps of all rows go to neighbouring words and queue (32 greedy
-// rows in 18 slices each 19.3 us, in 5 slices 10.1 us).
-constexpr int SLICE_MIN = 8192;
-constexpr int GREEDY_SLICES = 4;
-
+// A workgroup scans a row, or a slice of a long one: drawing the noise of a 151936-wide row (two logarithms and two
+// 64-bit products per value) takes one CU 70 us.  Slices of one row meet in out[row] itself: the key of the index that it
+// holds can be formed again from the logits, so a workgroup that found a better candidate replaces it with a
+// compare-and-swap (retried while others do the same; every retry means the row got better).  An index left there by an
+// earlier call is one more candidate of this row, anything else is no candidate, so nothing has to be cleared first.  No
+// scratch, and the result does not depend on the order: the largest key wins.
+// Measured, rows of 151936, one workgroup a row -> slices: one row greedy 16.4 -> 5.2 us, with noise 69 -> 9.3 us; 32 rows
+// 17.1 -> 8.3 and 70 -> 22 us, a third of them with noise 70 -> 13.8 us.
 __device__ __forceinline__ uint64_t mix64(uint64_t x) {  // SplitMix64 finaliser, as cpu/sample.zig:7-12
     x += 0x9E3779B97F4A7C15ull;
     x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -245,21 +240,23 @@ __device__ __forceinline__ uint64_t shfl_xor64(uint64_t x, int m) {
 template <bool GUMBEL>
 __device__ __forceinline__ uint64_t key_of(float x, int i, float temp, uint64_t rs) {
     if (GUMBEL) {
-        const uint64_t r = mix64(rs + (uint64_t)i);
+        const uint64_t r = mix64(rs + (uint32_t)i);
         const float u = ((float)(r >> 40) + 0.5f) * (1.0f / 16777216.0f);
         x = x / temp - logf(-logf(u));
     }
     return cand_key(x, i);
 }
 
-// The best key of one slice of a row for this lane.  The row is read in 16-byte vectors from its first aligned value on,
-// four per lane in flight; the first slice also takes the values before that, the last one those left at the end.
-template <bool GUMBEL>
+// The best key of one slice of a row for this lane.  The row is read in 16-byte vectors from its first aligned value on
+// (greedy four per lane in flight; with noise the arithmetic hides the read); the first slice also takes the values before
+// that, the last one those left at the end.
+template <bool GUMBEL, int THREADS>
 __device__ __forceinline__ uint64_t scan_slice(const bf16_t *row, int V, int slice, int slices, float temp,
                                                uint64_t rs) {
-    constexpr int U = 4;
+    constexpr int U = GUMBEL ? 1 : 4;
     const int head = min(V, (int)((16 - ((uintptr_t)row & 15)) & 15) / 2), vecs = (V - head) / 8;
-    const int per = (vecs + slices - 1) / slices, v0 = slice * per, v1 = min(vecs, v0 + per);
+    const int per = slices == 1 ? vecs : (vecs + slices - 1) / slices;
+    const int v0 = slice * per, v1 = min(vecs, v0 + per);
     uint64_t best = 0;
     auto take = [&](float x, int i) {
         const uint64_t k = key_of<GUMBEL>(x, i, temp, rs);
@@ -267,13 +264,13 @@ __device__ __forceinline__ uint64_t scan_slice(const bf16_t *row, int V, int sli
     };
     float top = -INFINITY;  // greedy: the value and index of this lane's best candidate
     int at = 0;
-    for (int v = v0 + threadIdx.x; v < v1; v += ROW_THREADS * U) {
+    for (int v = v0 + threadIdx.x; v < v1; v += THREADS * U) {
         u32x4_t raw[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) raw[u] = ld16(row + head + (long)min(v + u * ROW_THREADS, v1 - 1) * 8);
+        for (int u = 0; u < U; ++u) raw[u] = ld16(row + head + (long)min(v + u * THREADS, v1 - 1) * 8);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int vi = v + u * ROW_THREADS;
+            const int vi = v + u * THREADS;
             if (vi >= v1) break;
             float f[8];
             unpack_bf16x8(raw[u], f);
@@ -300,44 +297,45 @@ __device__ __forceinline__ uint64_t scan_slice(const bf16_t *row, int V, int sli
     return best;
 }
 
-__global__ void sample_start_kernel(int *out, int S) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < S) out[s] = 0;  // the scan's starting index, and the answer when no value is a candidate
-}
-
-// Workgroup (slice, row); slices == 1: the row's only one, which writes the result without looking at out.
-__global__ void __launch_bounds__(ROW_THREADS) sample_rows_kernel(int *out, const bf16_t *logits, const float *temps,
-                                                                   const uint64_t *seed, int V, int slices) {
-    const int s = blockIdx.x / slices, slice = blockIdx.x % slices;
+// CUT: workgroup (slice, row) of rows cut into noise_slices or, greedy ones, greedy_slices; else workgroup (row).
+template <int THREADS, bool CUT>
+__global__ void __launch_bounds__(THREADS) sample_rows_kernel(int *out, const bf16_t *logits, const float *temps,
+                                                               const uint64_t *seed, int V, int noise_slices,
+                                                               int greedy_slices) {
+    const int s = CUT ? blockIdx.y : blockIdx.x, slice = CUT ? blockIdx.x : 0;
     const float temp = temps[s];
     const bool gumbel = temp > 0.0f;
-    if (!gumbel) slices = (slices + GREEDY_SLICES - 1) / GREEDY_SLICES;
+    const int slices = !CUT ? 1 : gumbel ? noise_slices : greedy_slices;
     if (slice >= slices) return;
     const bf16_t *row = logits + (long)s * V;
     const uint64_t rs = gumbel ? mix64(*seed ^ ((uint64_t)s << 40)) : 0;
-    uint64_t best = gumbel ? scan_slice<true>(row, V, slice, slices, temp, rs)
-                           : scan_slice<false>(row, V, slice, slices, temp, 0);
+    uint64_t best = gumbel ? scan_slice<true, THREADS>(row, V, slice, slices, temp, rs)
+                           : scan_slice<false, THREADS>(row, V, slice, slices, temp, 0);
 #pragma unroll
     for (int m = 1; m < 64; m <<= 1) {
         const uint64_t o = shfl_xor64(best, m);
         best = o > best ? o : best;
     }
-    __shared__ uint64_t wave_best[ROW_THREADS / 64];
+    __shared__ uint64_t wave_best[THREADS / 64];
     if ((threadIdx.x & 63) == 0) wave_best[threadIdx.x >> 6] = best;
     __syncthreads();
     if (threadIdx.x != 0) return;
-    for (int w = 1; w < ROW_THREADS / 64; ++w) best = wave_best[w] > best ? wave_best[w] : best;
-    const int mine = best == 0 ? 0 : (int)~(uint32_t)best;
+    for (int w = 1; w < THREADS / 64; ++w) best = wave_best[w] > best ? wave_best[w] : best;
+    const int mine = best == 0 ? 0 : (int)~(uint32_t)best;  // 0: the scan's starting index, if no value is a candidate
     if (slices == 1) {
         out[s] = mine;
         return;
     }
     int cur = __hip_atomic_load(out + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (;;) {
-        const float x = bf2f(row[cur]);
-        const uint64_t k = gumbel ? key_of<true>(x, cur, temp, rs) : key_of<false>(x, cur, temp, 0);
-        if (best <= k || __hip_atomic_compare_exchange_strong(out + s, &cur, mine, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                              __HIP_MEMORY_SCOPE_AGENT))
+        uint64_t k = 0;
+        if ((unsigned)cur < (unsigned)V) {
+            const float x = bf2f(row[cur]);
+            k = gumbel ? key_of<true>(x, cur, temp, rs) : key_of<false>(x, cur, temp, 0);
+        }
+        if (best < k || (best == k && cur == mine) ||
+            __hip_atomic_compare_exchange_strong(out + s, &cur, mine, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT))
             return;
     }
 }
@@ -452,12 +450,29 @@ void hip_sample(int32_t *out_ids, const uint16_t *logits, const float *temps, co
         reject("hip_sample: V must be positive");
         return;
     }
-    // slices: enough workgroups to fill the chip eight times over (rows with noise take far longer than greedy ones)
-    int slices = std::max(1, std::min(V / SLICE_MIN, 8 * llmgen_num_cus() / S));
-    if (slices > 1 && !on_this_device(out_ids)) slices = 1;  // one workgroup a row, which writes its id with a plain store
-    if (slices > 1) sample_start_kernel<<<blocks_for(S, 256), 256, 0, g_llmgen_stream>>>(out_ids, S);
-    sample_rows_kernel<<<(unsigned)S * slices, ROW_THREADS, 0, g_llmgen_stream>>>(out_ids, logits, temps, seed, V,
-                                                                                   slices);
+    // Slices of rows with noise: two workgroups a CU at most, and 8192 values in one at least.  Beyond a row for every
+    // other CU only long rows gain (128 rows of 16384: 9.9 -> 8.3 us; 256 rows of 32000 would take 19.1 in two slices, not
+    // 17.8 us; 256 rows of 151936, a third with noise: 72 -> 40 us).  Greedy rows are a plain read, and their slices queue
+    // at the compare-and-swaps, since the words of all rows are neighbours (256 rows of 65536: 5.8 us whole, 7.4 in two
+    // slices, 13.3 in four): fewer and longer slices.
+    const int cus = llmgen_num_cus();
+    int n = std::max(1, std::min({16, V / 8192, 2 * cus / S}));
+    if (S > cus / 2 && V < 49152) n = 1;
+    if (n > 1 && !on_this_device(out_ids)) n = 1;  // one workgroup a row, which writes its id with a plain store
+    const int g = std::max(1, std::min({n, V / 32768, cus / S}));
+    auto launch = [&](auto kernel, dim3 grid, int threads) {
+        kernel<<<grid, threads, 0, g_llmgen_stream>>>(out_ids, logits, temps, seed, V, n, g);
+    };
+    // Lanes for a vector each; where a CU holds several short rows, half as many with two (700 rows of 8192, greedy: 5.6 us
+    // with 1024 lanes, 4.0 with 512; 1100 rows of 16384 with noise 36.0 and 36.5).
+    if (n > 1)
+        launch(sample_rows_kernel<1024, true>, dim3(n, S), 1024);
+    else if (V <= 2048)
+        launch(sample_rows_kernel<256, false>, S, 256);
+    else if (V <= 4096 || (V <= 8192 && S > cus))
+        launch(sample_rows_kernel<512, false>, S, 512);
+    else
+        launch(sample_rows_kernel<1024, false>, S, 1024);
 }
 
 }  // extern "C"

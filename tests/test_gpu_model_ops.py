@@ -159,3 +159,26 @@ def test_mlp_and_sampling_captured(gpu):
                 assert torch.equal(got, want)
     finally:
         L.hip_graph_destroy(graph)
+
+
+# (S, V) at the edges of the launch rule (256 CUs): 256, 512 and 1024 lanes for whole rows, cut rows with and without cut
+# greedy ones, the most slices, and a row for every other CU and beyond
+@pytest.mark.parametrize("S,V", [(2, 2048), (3, 2049), (257, 8190), (5, 4097), (40, 16384), (2, 70001), (1, 131072),
+                                 (128, 16390), (129, 49151), (129, 49152), (200, 65537)])
+def test_sample_any_previous_ids(gpu, S, V):
+    """Cut rows meet in out_ids, whatever it holds before the call: rubbish, the answer, another index, an index whose
+    logit is no candidate."""
+    rng = np.random.default_rng(S * 3 + V)
+    lg = draw(rng, S, V)
+    lg[0] = 0xFF80  # no candidate: index 0
+    lg[-1, 5] = 0x7FC0
+    temps = np.where(np.arange(S) % 2 == 1, 0.9, 0.0).astype(np.float32)
+    seed = torch.tensor([31], dtype=torch.int64, device="cuda")
+    ref = O.sample(lg, temps, seed=31)
+    ld, td = up(lg), up(temps)
+    for before in (-1, 2**31 - 1, V, V - 1, 5, ref):
+        out = torch.tensor(np.broadcast_to(before, S).astype(np.int32), device="cuda")
+        lib().hip_sample(out.data_ptr(), ld.data_ptr(), td.data_ptr(), seed.data_ptr(), S, V, None)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.cpu().numpy(), ref)
+    assert lib().hip_last_error() == 0
