@@ -32,7 +32,7 @@ extern "C" {
 void hip_embedding(uint16_t *out, const int32_t *ids, const uint16_t *weight, int T, int H);
 
 /* out [rows, D] bf16 = bf16(bf16(x * scale) * w), scale = 1 / sqrt(sum(x^2) / D + eps), the sum taken in index
- * order in f32.  x bf16, w f32 [D] (GGUF norm gains are f32).  D % 8 == 0 and D <= 8192. */
+ * order in f32.  x bf16, 16-byte aligned, w f32 [D] (GGUF norm gains are f32).  D % 8 == 0 and D <= 8192. */
 void hip_rmsnorm(uint16_t *out, const uint16_t *x, const float *w, long rows, int D, float eps);
 
 /* y [M, N] = x [M, K] * w [N, K]^T with f32 accumulation over k = 0..K-1 in order; y is bf16 (RNE) or, with
@@ -66,7 +66,8 @@ void hip_gather_rows(uint16_t *out, const uint16_t *x, const int32_t *idx, int S
 
 /* out_ids [S] = argmax over logits [S, V] bf16 per row: greedy when temps[s] <= 0 (the first index of the maximum),
  * else Gumbel-max of logits / temp with splitmix64 noise keyed by (*seed, s, index).  out_ids may also be pinned host
- * memory; in memory of the device, several workgroups share a long row and its word.  No scratch is used:
+ * memory; in memory of the device, several workgroups share a long row and its word, whatever that holds before the
+ * call.  No scratch is used:
  * hip_sample_scratch_bytes returns 0 and scratch may be NULL (both kept for the reference's argument list). */
 void hip_sample(int32_t *out_ids, const uint16_t *logits, const float *temps, const uint64_t *seed, int S, int V,
                 void *scratch);

@@ -38,6 +38,10 @@ __global__ void embedding_kernel(bf16_t *out, const int *ids, const bf16_t *w, i
 // Measured, D = 1024: 32 rows 14.7 -> 5.2 us, 2051 rows 36 -> 7.4 us (before: one lane of a wave formed each square and
 // sum).
 constexpr int NORM_MAX_D = 8192;
+// The output and the gains may lie at any value's address (x is 16-byte aligned), which these types tell the compiler; it
+// moves them as whole vectors all the same.
+typedef u32x4_t u32x4_any_t __attribute__((aligned(2)));
+typedef f32x4_t f32x4_any_t __attribute__((aligned(4)));
 template <int R>
 __global__ void __launch_bounds__(64) rmsnorm_kernel(bf16_t *out, const bf16_t *x, const float *w, long rows, int D,
                                                       float eps) {
@@ -71,8 +75,8 @@ __global__ void __launch_bounds__(64) rmsnorm_kernel(bf16_t *out, const bf16_t *
 #pragma unroll
         for (int i = 0; i < KEEP; ++i)
             if (sub + i * L < chunks) {
-                gain[i][0] = *reinterpret_cast<const f32x4_t *>(w + (sub + i * L) * 8);
-                gain[i][1] = *reinterpret_cast<const f32x4_t *>(w + (sub + i * L) * 8 + 4);
+                gain[i][0] = *reinterpret_cast<const f32x4_any_t *>(w + (sub + i * L) * 8);
+                gain[i][1] = *reinterpret_cast<const f32x4_any_t *>(w + (sub + i * L) * 8 + 4);
             }
 #pragma unroll
         for (int i = 0; i < KEEP; ++i)
@@ -123,7 +127,7 @@ __global__ void __launch_bounds__(64) rmsnorm_kernel(bf16_t *out, const bf16_t *
 #pragma unroll
         for (int h = 0; h < 4; ++h)
             o[h] = pack_bf16x2(bf2f(f2bf(f[2 * h] * scale)) * g[2 * h], bf2f(f2bf(f[2 * h + 1] * scale)) * g[2 * h + 1]);
-        *reinterpret_cast<u32x4_t *>(out + r * D + c * 8) = o;
+        *reinterpret_cast<u32x4_any_t *>(out + r * D + c * 8) = o;
     };
     if (kept) {
 #pragma unroll
@@ -132,8 +136,8 @@ __global__ void __launch_bounds__(64) rmsnorm_kernel(bf16_t *out, const bf16_t *
     } else {
 #pragma unroll 4
         for (int c = sub; c < chunks; c += L)
-            finish(ld16(xr + c * 8), *reinterpret_cast<const f32x4_t *>(w + c * 8),
-                   *reinterpret_cast<const f32x4_t *>(w + c * 8 + 4), c);
+            finish(ld16(xr + c * 8), *reinterpret_cast<const f32x4_any_t *>(w + c * 8),
+                   *reinterpret_cast<const f32x4_any_t *>(w + c * 8 + 4), c);
     }
 }
 

@@ -182,3 +182,16 @@ def test_sample_any_previous_ids(gpu, S, V):
         torch.cuda.synchronize()
         np.testing.assert_array_equal(out.cpu().numpy(), ref)
     assert lib().hip_last_error() == 0
+
+
+@pytest.mark.parametrize("rows,D", [(3, 1000), (5, 8192), (2051, 264), (4099, 136), (8195, 128)])
+@pytest.mark.parametrize("gains,offset", [(1, 0), (2, 3), (3, 1)])
+def test_rmsnorm_gains_and_output_at_any_address(gpu, rows, D, gains, offset):
+    rng = np.random.default_rng(rows * gains)
+    x, g = draw(rng, rows, D, std=2.0), (1 + 0.1 * rng.standard_normal(D)).astype(np.float32)
+    out = torch.zeros(rows * D + offset + 8, dtype=torch.int16, device="cuda")
+    xd, gd = up(x), torch.cat([torch.zeros(gains, device="cuda"), up(g)])
+    lib().hip_rmsnorm(out.data_ptr() + 2 * offset, xd.data_ptr(), gd.data_ptr() + 4 * gains, rows, D, 1e-6)
+    got = down(out)
+    np.testing.assert_array_equal(got[offset:offset + rows * D].reshape(rows, D), O.rmsnorm(x, g, 1e-6))
+    assert not got[:offset].any() and not got[offset + rows * D:].any()
