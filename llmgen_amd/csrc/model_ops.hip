@@ -159,8 +159,9 @@ __global__ void rope_kernel(bf16_t *out, const bf16_t *x, const float *cos_t, co
 }
 
 // ---------------------------------------------------------------------------------------------- elementwise
-// Streams of bf16: eight values per lane and 16-byte accesses where every pointer allows them, the last n % 8 values
-// (or all of them) one by one.
+// Streams of bf16: eight values per lane and 16-byte accesses where every pointer allows them, the last n % 8 values one by
+// one; else a value per lane in a kernel of its own, which has none of the split's arithmetic (2^24 values, add: 25.5 us, 26.8
+// as the vector kernel's tail).
 struct SiluOp {
     __device__ __forceinline__ float operator()(float v, float) const { return v / (1.0f + expf(-v)); }
 };
@@ -190,6 +191,13 @@ __global__ void __launch_bounds__(256) elementwise_kernel(bf16_t *out, const bf1
         const size_t e = vecs * 8 + (i - vecs);
         if (e < n) out[e] = f2bf(op(bf2f(a[e]), bf2f(b[e])));
     }
+}
+
+template <class Op>
+__global__ void __launch_bounds__(256) elementwise_single_kernel(bf16_t *out, const bf16_t *a, const bf16_t *b, size_t n,
+                                                                 Op op) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = f2bf(op(bf2f(a[i]), bf2f(b[i])));
 }
 
 __global__ void gather_rows_kernel(bf16_t *out, const bf16_t *x, const int *idx, int S, int H) {
@@ -367,8 +375,11 @@ bool on_this_device(const void *p) {
 template <class Op>
 void elementwise(bf16_t *out, const bf16_t *a, const bf16_t *b, size_t n, Op op) {
     if (n == 0) return;
-    const bool aligned = (((uintptr_t)out | (uintptr_t)a | (uintptr_t)b) & 15) == 0;
-    const size_t vecs = aligned ? n / 8 : 0;
+    if (((uintptr_t)out | (uintptr_t)a | (uintptr_t)b) & 15) {
+        elementwise_single_kernel<<<blocks_for(n, 256), 256, 0, g_llmgen_stream>>>(out, a, b, n, op);
+        return;
+    }
+    const size_t vecs = n / 8;
     elementwise_kernel<<<blocks_for(vecs + (n - vecs * 8), 256), 256, 0, g_llmgen_stream>>>(out, a, b, vecs, n, op);
 }
 
