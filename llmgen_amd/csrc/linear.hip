@@ -141,7 +141,7 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64, PW ? 1 : 2) linear_kernel
     __shared__ __attribute__((aligned(16))) float lds[2][T::ROWS * T::STRIDE];
     __shared__ int flag[3];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) flag[0] = 0;
+    if (tid < 2) flag[tid] = 0;
     // tiles in order of columns, each XCD (block index mod 8) a contiguous range of them
     const int tiles = gridDim.x;
     const int per = tiles >> 3, rem = tiles & 7, xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
@@ -306,7 +306,8 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64, PW ? 1 : 2) linear_kernel
     };
     // Step i: the products of chunk i, the fragments of chunk i + 1, the staging of chunk i + 2, the loads of chunk
     // i + 2 + PF.  Returns whether a value lies outside its window (then the sums are of no use): asked after the first
-    // two chunks and at the end.
+    // two chunks (flag[0]) and at the end (flag[1]: with a short K a fast wave is at the last steps, and sets its flag, while
+    // a slow one has yet to read the first, and both must take the same way past the barriers).
     const int chunks = full + (tail > 0);
     auto flagged = [&](int i) { return __builtin_amdgcn_readfirstlane(flag[i]) != 0; };
     auto run = [&](auto stager, auto multiplier) {
@@ -367,10 +368,10 @@ __global__ void __launch_bounds__((WM * WN + PW) * 64, PW ? 1 : 2) linear_kernel
                     if (i + p + 2 < chunks) stage(raw[(p + 2) % PF], p & 1);
                 if constexpr (C) compute(p & 1);
                 if constexpr (S)
-                    if (bad) flag[0] = 1;
+                    if (bad) flag[1] = 1;
                 __syncthreads();
             }
-        return flagged(0);
+        return flagged(1);
     };
     const bool multiplier = !PW || __builtin_amdgcn_readfirstlane(wave) < T::WAVES, stager = !PW || !multiplier;
     bool again;

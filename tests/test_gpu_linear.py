@@ -186,3 +186,15 @@ def test_linear3_wide_equals_single_products(gpu, M, Ns):
         got, ref = y.cpu().numpy(), run(x, w, False)[:, :n] if n else np.zeros((M, 0), np.uint16)
         assert (got[M * n:] == 77).all()
         np.testing.assert_array_equal(got[:M * n].view(np.uint16).reshape(M, n), ref)
+
+
+@pytest.mark.parametrize("M,N,K,chunk", LOOPS)
+@pytest.mark.parametrize("chunks", [3, 4])
+def test_linear_few_chunks_outside_the_exact_window(gpu, M, N, K, chunk, chunks):
+    """Too short a K for the pipelined loop, and in every tile a value outside the window from the third chunk on: the waves
+    of a workgroup learn of it in the last steps, and only there."""
+    rng = np.random.default_rng(M + chunks)
+    K = (chunks - 1) * chunk + 24
+    x, w = draw(rng, M, K), draw(rng, N, K, std=0.05)
+    x[::16, 2 * chunk + 5] = O.f32_to_bf16(np.array([2.0**-70], np.float32))[0]
+    check(x, w, y_f32=True)
