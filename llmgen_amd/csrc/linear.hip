@@ -133,9 +133,11 @@ struct LinTile {
 
 // "At least two waves a SIMD" keeps the sums in ordinary registers, where the VALU adds to them without moves.  Not so in
 // the kernels with producer waves, which are 2 % faster without it (32 x 1024 x 3072: 15.9 and 16.3 us; with values outside
-// the window throughout 83 and 58 us).
+// the window throughout 83 and 58 us).  32 x 32 tiles, many to a CU, fit four waves a SIMD, as many as the LDS holds
+// (100 x 9001 x 200: 12.4 us, 13.4 with three).
 template <int MT, int NT, int WM, int WN, int PW, int KC, int PF>
-__global__ void __launch_bounds__((WM * WN + PW) * 64, PW ? 1 : 2) linear_kernel(const LinArgs a) {
+__global__ void __launch_bounds__((WM * WN + PW) * 64, PW ? 1 : WM * WN * MT * NT == 4 ? 4 : 2)
+    linear_kernel(const LinArgs a) {
     using T = LinTile<MT, NT, WM, WN, PW, KC>;
     static_assert(PF % 2 == 0, "chunk parity names the LDS buffer");
     __shared__ __attribute__((aligned(16))) float lds[2][T::ROWS * T::STRIDE];
