@@ -578,6 +578,44 @@ __global__ void __launch_bounds__(256, 2) linear_stream_kernel(const LinArgs a) 
         if (half * 4 + r < a.M) lin_put(a, out, half * 4 + r, n, acc[r]);
 }
 
+// K of 8 and 16 (a low-rank update): nothing to pipeline, and the tiles would stage and multiply mostly zeros.  Bound by
+// latencies and the store of y: a lane owns a column, its row of w and SHORT_ROWS rows of x are loaded at once, then
+// multiplies and adds as the reference's.  1 x 1000 x 8: 1.8 us (tiles 4.0, the multiply-add kernel before them 3.0),
+// 300 x 4096 x 16 3.9 (6.9, 6.0), 2051 x 4096 x 8 10.0 (17.0, 13.3); from K = 24 on the tiles are the faster.
+constexpr int SHORT_ROWS = 8, SHORT_COLS = 256;
+template <int K>
+__global__ void __launch_bounds__(SHORT_COLS) linear_short_kernel(const LinArgs a) {
+    int n0;
+    const LinOut out = lin_out(a, blockIdx.x / a.tiles_m, SHORT_COLS, n0);
+    const int n = n0 + threadIdx.x, m0 = blockIdx.x % a.tiles_m * SHORT_ROWS;
+    if (n >= out.N) return;
+    u32x4_t wr[K / 8], xr[SHORT_ROWS][K / 8];
+#pragma unroll
+    for (int i = 0; i < K / 8; ++i) {
+        wr[i] = ld16(out.w + (long)n * K + i * 8);
+#pragma unroll
+        for (int r = 0; r < SHORT_ROWS; ++r) xr[r][i] = ld16(a.x + (long)min(m0 + r, a.M - 1) * K + i * 8);
+    }
+    float w[K], x[K];
+#pragma unroll
+    for (int i = 0; i < K / 8; ++i) unpack_bf16x8(wr[i], w + i * 8);
+#pragma unroll
+    for (int r = 0; r < SHORT_ROWS; ++r) {
+        if (m0 + r >= a.M) return;
+#pragma unroll
+        for (int i = 0; i < K / 8; ++i) unpack_bf16x8(xr[r][i], x + i * 8);
+        float sum = 0.f;
+#pragma unroll
+        for (int k = 0; k < K; ++k) sum = sum + x[k] * w[k];
+        lin_put(a, out, m0 + r, n, sum);
+    }
+}
+template <int K>
+void linear_short_launch(LinArgs a) {
+    a.tiles_m = (a.M + SHORT_ROWS - 1) / SHORT_ROWS;
+    linear_short_kernel<K><<<(unsigned)(a.tiles_m * lin_cols(a, SHORT_COLS)), SHORT_COLS, 0, g_llmgen_stream>>>(a);
+}
+
 // Tiles of the throughput-bound sizes.  A launch takes about as long as the CU with the most tiles:
 // ceil(tiles / CUs) * blocks of a tile / rate, where `rate` is the share of the matrix cores' peak that the tile
 // reached on sizes it fits (launch time taken off): 0.68 for 32 x 32 (631 x 1024 x 3072: 47.8 us; 350 x 1024 x 3072:
@@ -599,6 +637,8 @@ const LinChoice LIN_CHOICES[] = {{32, 32, 0.68f, linear_launch<1, 1, 2, 2, 0, 64
 void linear_dispatch(const LinArgs &a) {
     const long blocks = (long)((a.M + 15) / 16) * lin_cols(a, 16);
     const int cus = llmgen_num_cus();
+    if (a.K == 8) return linear_short_launch<8>(a);
+    if (a.K == 16) return linear_short_launch<16>(a);
     // At most one 16 x 16 block per CU: one block and three staging waves a workgroup (7.8 us at 1 x 1024 x 1024,
     // 17.3 us at 32 x 1024 x 3072; 32 x 32 tiles 9.5 and 26 us).
     if (blocks <= cus) return linear_launch<1, 1, 1, 1, 3, 128, 2>(a);

@@ -198,3 +198,45 @@ def test_linear_few_chunks_outside_the_exact_window(gpu, M, N, K, chunk, chunks)
     x, w = draw(rng, M, K), draw(rng, N, K, std=0.05)
     x[::16, 2 * chunk + 5] = O.f32_to_bf16(np.array([2.0**-70], np.float32))[0]
     check(x, w, y_f32=True)
+
+
+# the kernel of K = 8 and 16: eight rows and 256 columns a workgroup, an edge on either side; K = 24 is the first on tiles
+@pytest.mark.parametrize("M,N", [(1, 1), (7, 255), (8, 256), (9, 257), (17, 1030), (2051, 4096)])
+@pytest.mark.parametrize("K", [8, 16, 24])
+@pytest.mark.parametrize("special", [False, True])
+def test_linear_short_k(gpu, M, N, K, special):
+    rng = np.random.default_rng(M + N + K)
+    x, w = draw(rng, M, K), draw(rng, N, K)
+    if special:
+        for a in (x, w):
+            at = rng.integers(0, a.size, 1 + a.size // 50)
+            a.reshape(-1)[at] = rng.choice(np.array([0, 0x8000, 1, 0x8001, 0x1000, 0x7F00, 0xFF7F, 0x7F80, 0x7FC0], np.uint16),
+                                           at.size)
+    check(x, w, y_f32=True, offset=1)
+    check(x, w, y_f32=False, offset=M % 2)
+
+
+@pytest.mark.parametrize("K", [8, 16])
+@pytest.mark.parametrize("M,Ns", [(1, (300, 1, 0)), (13, (256, 257, 33)), (300, (0, 2000, 600))])
+def test_linear3_and_add_of_short_k(gpu, K, M, Ns):
+    rng = np.random.default_rng(K + M)
+    x, ws = draw(rng, M, K), [draw(rng, max(n, 1), K) for n in Ns]
+    xd, wd = torch.from_numpy(x.view(np.int16)).cuda(), [torch.from_numpy(w.view(np.int16)).cuda() for w in ws]
+    ys = [torch.full((M * n + 8,), 77, dtype=torch.int16, device="cuda") for n in Ns]
+    args = [a for y, w, n in zip(ys, wd, Ns) for a in ((y.data_ptr(), w.data_ptr(), n) if n else (None, None, 0))]
+    lib().hip_linear3(*args, xd.data_ptr(), M, K)
+    refs = [O.linear(x, w)[:, :n].reshape(-1) for w, n in zip(ws, Ns)]
+    sums = []
+    for w, n, ref in zip(wd, Ns, refs):
+        res = draw(rng, M * n)
+        rd = torch.from_numpy(res.view(np.int16)).cuda()
+        if n:
+            lib().hip_linear_add(rd.data_ptr(), rd.data_ptr(), xd.data_ptr(), w.data_ptr(), M, n, K)
+        sums.append((rd, O.add(res, ref) if n else res))
+    torch.cuda.synchronize()
+    assert lib().hip_last_error() == 0
+    for y, ref, (rd, total) in zip(ys, refs, sums):
+        got = y.cpu().numpy()
+        assert (got[ref.size:] == 77).all()
+        np.testing.assert_array_equal(got[:ref.size].view(np.uint16), ref)
+        np.testing.assert_array_equal(rd.cpu().numpy().view(np.uint16), total)
