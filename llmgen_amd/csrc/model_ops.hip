@@ -224,8 +224,8 @@ __global__ void gather_rows_kernel(bf16_t *out, const bf16_t *x, const int *idx,
 // compare-and-swap (retried while others do the same; every retry means the row got better).  An index left there by an
 // earlier call is one more candidate of this row, anything else is no candidate, so nothing has to be cleared first.  No
 // scratch, and the result does not depend on the order: the largest key wins.
-// Measured, rows of 151936, one workgroup a row -> slices: one row greedy 16.4 -> 5.2 us, with noise 69 -> 9.3 us; 32 rows
-// 17.1 -> 8.3 and 70 -> 22 us, a third of them with noise 70 -> 13.8 us.
+// Measured, rows of 151936, one workgroup a row -> slices: one row greedy 16.2 -> 4.2 us, with noise 69 -> 5.2 us; 32 rows
+// 17.0 -> 4.4 and 70 -> 12.3 us, a third of them with noise 70 -> 9.2 us.
 __device__ __forceinline__ uint64_t mix64(uint64_t x) {  // SplitMix64 finaliser, as cpu/sample.zig:7-12
     x += 0x9E3779B97F4A7C15ull;
     x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -309,12 +309,15 @@ __device__ __forceinline__ uint64_t scan_slice(const bf16_t *row, int V, int sli
     return best;
 }
 
-// CUT: workgroup (slice, row) of rows cut into noise_slices or, greedy ones, greedy_slices; else workgroup (row).
+// CUT: S rows cut into noise_slices workgroups, of which greedy rows use the first greedy_slices; else a workgroup a row.
+// All first slices come first, then all second ones, each time one row further on: workgroups go to the XCDs in turn, and
+// so the slices in use, and those of one row, lie on all of them (slice by slice of a row, two slices of which greedy rows
+// use one left every other XCD idle: 256 greedy rows of 65536 9.4 us, so 5.8).
 template <int THREADS, bool CUT>
 __global__ void __launch_bounds__(THREADS) sample_rows_kernel(int *out, const bf16_t *logits, const float *temps,
                                                                const uint64_t *seed, int V, int noise_slices,
-                                                               int greedy_slices) {
-    const int s = CUT ? blockIdx.y : blockIdx.x, slice = CUT ? blockIdx.x : 0;
+                                                               int greedy_slices, int S) {
+    const int slice = CUT ? blockIdx.x / S : 0, s = CUT ? (blockIdx.x + slice) % S : blockIdx.x;
     const float temp = temps[s];
     const bool gumbel = temp > 0.0f;
     const int slices = !CUT ? 1 : gumbel ? noise_slices : greedy_slices;
@@ -465,26 +468,29 @@ void hip_sample(int32_t *out_ids, const uint16_t *logits, const float *temps, co
         reject("hip_sample: V must be positive");
         return;
     }
-    // Slices of rows with noise: two workgroups a CU at most, and 8192 values in one at least.  Beyond a row for every
-    // other CU only long rows gain (128 rows of 16384: 9.9 -> 8.3 us; 256 rows of 32000 would take 19.1 in two slices, not
-    // 17.8 us; 256 rows of 151936, a third with noise: 72 -> 40 us).  Greedy rows are a plain read, and their slices queue
-    // at the compare-and-swaps, since the words of all rows are neighbours (256 rows of 65536: 5.8 us whole, 7.4 in two
-    // slices, 13.3 in four): fewer and longer slices.
+    // Slices of rows with noise: 2048 values in one at least, four vectors a lane of 512, and 8 to 16 slices, few rows 32.
+    // The host does not know which rows have noise: a third of them fills the chip evenly only in small slices (200 rows
+    // of 151936, a third with noise: 31 us in 16 slices, 67 in two of 1024 lanes, 72 whole; all of them: 55, 68 and 73 us).  Whole rows
+    // where many rows fill it anyway, and where slices would be short (256 rows of 12000 with noise: 8.0 us whole, 8.9 in
+    // four; 256 rows of 16384: 10.1 and 10.5 us, but a third of them 9.8 and 7.1).
+    // Greedy rows are a plain read, and their slices queue at the compare-and-swaps, since the words of all rows are
+    // neighbours: one, or a few of 16384 values at least (32 rows of 151936: 9.9 us in one, 6.3 in two, 4.6 in four; 200 rows
+    // of 65536: 6.1, 5.9, 6.0).
     const int cus = llmgen_num_cus();
-    int n = std::max(1, std::min({16, V / 8192, 2 * cus / S}));
-    if (S > cus / 2 && V < 49152) n = 1;
+    int n = std::min(V / 2048, S <= cus / 8 ? 32 : std::max(8, std::min(16, V / 4096)));
+    n = V <= 8192 || (V < 16384 && S > cus / 2) ? 1 : std::max(1, std::min(n, (V < 24576 ? 4 : 16) * cus / S));
     if (n > 1 && !on_this_device(out_ids)) n = 1;  // one workgroup a row, which writes its id with a plain store
-    const int g = std::max(1, std::min({n, V / 32768, cus / S}));
-    auto launch = [&](auto kernel, dim3 grid, int threads) {
-        kernel<<<grid, threads, 0, g_llmgen_stream>>>(out_ids, logits, temps, seed, V, n, g);
+    const int g = std::min(n, V < 65536 ? 1 : S <= cus * 5 / 8 ? 4 : 2);
+    auto launch = [&](auto kernel, int grid, int threads) {
+        kernel<<<grid, threads, 0, g_llmgen_stream>>>(out_ids, logits, temps, seed, V, n, g, S);
     };
-    // Lanes for a vector each; where a CU holds several short rows, half as many with two (700 rows of 8192, greedy: 5.6 us
-    // with 1024 lanes, 4.0 with 512; 1100 rows of 16384 with noise 36.0 and 36.5).
+    // Whole rows: lanes for a vector each; where a CU holds several rows, at most 512 of them (700 rows of 12000, a third
+    // with noise: 9.3 us, with 1024 lanes 14.0, all with noise 18.2 and 17.6).
     if (n > 1)
-        launch(sample_rows_kernel<1024, true>, dim3(n, S), 1024);
+        launch(sample_rows_kernel<512, true>, n * S, 512);
     else if (V <= 2048)
         launch(sample_rows_kernel<256, false>, S, 256);
-    else if (V <= 4096 || (V <= 8192 && S > cus))
+    else if (V <= 4096 || S > cus)
         launch(sample_rows_kernel<512, false>, S, 512);
     else
         launch(sample_rows_kernel<1024, false>, S, 1024);

@@ -195,3 +195,27 @@ def test_rmsnorm_gains_and_output_at_any_address(gpu, rows, D, gains, offset):
     got = down(out)
     np.testing.assert_array_equal(got[offset:offset + rows * D].reshape(rows, D), O.rmsnorm(x, g, 1e-6))
     assert not got[:offset].any() and not got[offset + rows * D:].any()
+
+
+# the edges of the rule for slices (256 CUs): cut from 8193 values, beyond 128 rows from 16384 on; 32 slices for up to 32
+# rows; four greedy slices for up to 160 rows from 65536 values on, else two; whole rows again beyond 1024 and 4096 rows
+@pytest.mark.parametrize("S,V", [(1, 8192), (3, 8193), (128, 8193), (129, 16383), (129, 16384), (32, 65536), (33, 65535), (1, 131071),
+                                 (160, 65536), (161, 65536), (300, 24575), (300, 24576), (1025, 16384), (1025, 24576), (4097, 8200)])
+def test_sample_slices_rule_edges(gpu, S, V):
+    """Every row holds its largest value twice, in two slices; a row without a candidate and one with NaN among them."""
+    rng = np.random.default_rng(S + 2 * V)
+    lg = np.broadcast_to(draw(rng, 1, V + 4096), (S, V + 4096))  # rows: one stream from another start each
+    lg = np.stack([row[i % 4096:i % 4096 + V] for i, row in enumerate(lg)])
+    for i, at in enumerate(rng.integers(0, V // 2, S)):
+        lg[i, [at, V - 1 - at % 7]] = 0x4110  # 9.0
+    lg[-1] = 0xFF80
+    lg[S // 2, 0] = 0x7FC0
+    temps = np.where(np.arange(S) % 5 == 1, 0.9, 0.0).astype(np.float32)
+    seed = torch.tensor([3], dtype=torch.int64, device="cuda")
+    ref = O.sample(lg, temps, seed=3)
+    ld, td, out = up(lg), up(temps), torch.full((S,), -5, dtype=torch.int32, device="cuda")
+    for _ in range(2):
+        lib().hip_sample(out.data_ptr(), ld.data_ptr(), td.data_ptr(), seed.data_ptr(), S, V, None)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.cpu().numpy(), ref)
+    assert lib().hip_last_error() == 0
