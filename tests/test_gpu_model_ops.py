@@ -219,3 +219,44 @@ def test_sample_slices_rule_edges(gpu, S, V):
         torch.cuda.synchronize()
         np.testing.assert_array_equal(out.cpu().numpy(), ref)
     assert lib().hip_last_error() == 0
+
+
+# a value per lane up to 65536 values, vectors of eight beyond, where all three addresses allow them (offset 8 does)
+@pytest.mark.parametrize("n", [65535, 65536, 65537, 65544, 70007, 300001])
+@pytest.mark.parametrize("offset", [0, 1, 8])
+def test_elementwise_long_streams(gpu, n, offset):
+    rng = np.random.default_rng(n)
+    a, b = draw(rng, n, std=4.0), draw(rng, n, std=2.0)
+    ad, bd = (torch.cat([torch.zeros(offset, dtype=torch.int16, device="cuda"), up(t)]) for t in (a, b))
+    for name, ref in (("add", O.add(a, b)), ("mul", O.mul(a, b)), ("silu_mul", None), ("silu", None)):
+        out = torch.zeros(n + offset + 16, dtype=torch.int16, device="cuda")
+        args = [t.data_ptr() + 2 * offset for t in ((out, ad) if name == "silu" else (out, ad, bd))]
+        getattr(lib(), "hip_" + name)(*args, n)
+        got = down(out)
+        assert not got[:offset].any() and not got[offset + n:].any()
+        np.testing.assert_array_equal(got[offset:offset + n], silu(a, b if name == "silu_mul" else None) if ref is None else ref)
+
+
+def silu(bits, up_bits=None):
+    """x / (1 + exp(-x)) with exp rounded once to f32, rounded to bf16; times ``up_bits``, rounded again."""
+    v = O.bf16_to_f32(bits)
+    with np.errstate(all="ignore"):
+        s = O.f32_to_bf16(v / (np.float32(1) + np.exp(-v.astype(np.float64)).astype(np.float32)))
+        return s if up_bits is None else O.f32_to_bf16(O.bf16_to_f32(s) * O.bf16_to_f32(up_bits))
+
+
+@pytest.mark.parametrize("copies", [1, 2])  # a value per lane, vectors
+def test_silu_and_silu_mul_every_gate(gpu, copies):
+    """All 65536 gates, in both kernels of both ops, against the form with a double exp rounded once."""
+    gates = np.tile(np.arange(65536, dtype=np.uint32).astype(np.uint16), copies)
+    gd, out = up(gates), torch.zeros(gates.size, dtype=torch.int16, device="cuda")
+    for factor in (None, 1.0, -0.7109375, 3.0e38, 2.0**-130):
+        ud = None if factor is None else O.f32_to_bf16(np.full(gates.size, factor, np.float32))
+        if ud is None:
+            lib().hip_silu(out.data_ptr(), gd.data_ptr(), gates.size)
+        else:
+            lib().hip_silu_mul(out.data_ptr(), gd.data_ptr(), up(ud).data_ptr(), gates.size)
+        got, ref = down(out), silu(gates, ud)
+        nan = (ref & 0x7FFF) > 0x7F80
+        np.testing.assert_array_equal((got & 0x7FFF) > 0x7F80, nan)
+        np.testing.assert_array_equal(got[~nan], ref[~nan])
