@@ -409,8 +409,9 @@ void hip_rmsnorm(uint16_t *out, const uint16_t *x, const float *w, long rows, in
         return;
     }
     // Rows per wave: as many as leave a wave for every SIMD (a SIMD runs two chains no faster than one after the
-    // other) while 8 waves' rows still fit a CU's LDS (9000 x 1024: 4 rows a wave 16.8 us, 8 rows 21.4 us; 3000 x 2048:
-    // 2 rows 14.0 us, 1 row 17.6 us).
+    // other) while the rows of 7 or 8 waves still fit a CU's LDS (8193 x 1024: 4 rows a wave 13.2 us, 8 rows 20.0 us; 3000 x
+    // 2048: 2 rows 13.6 us, 1 row 20.4 us; 8193 x 2560: 47 and 57 us; 8193 x 4096, where 2 rows a wave leave room for 4
+    // waves: 100 and 88 us).
     const long simds = 4L * llmgen_num_cus();
     auto launch = [&](auto kernel, int R) {
         kernel<<<(unsigned)((rows + R - 1) / R), 64, (size_t)R * (D + 4) * 4, g_llmgen_stream>>>(out, x, w, rows, D, eps);
@@ -419,7 +420,7 @@ void hip_rmsnorm(uint16_t *out, const uint16_t *x, const float *w, long rows, in
         launch(rmsnorm_kernel<8>, 8);
     else if (rows >= 4 * simds && D <= 1024)
         launch(rmsnorm_kernel<4>, 4);
-    else if (rows >= 2 * simds && D <= 4096)
+    else if (rows >= 2 * simds && D <= 2560)
         launch(rmsnorm_kernel<2>, 2);
     else
         launch(rmsnorm_kernel<1>, 1);

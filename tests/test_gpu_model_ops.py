@@ -260,3 +260,14 @@ def test_silu_and_silu_mul_every_gate(gpu, copies):
         nan = (ref & 0x7FFF) > 0x7F80
         np.testing.assert_array_equal((got & 0x7FFF) > 0x7F80, nan)
         np.testing.assert_array_equal(got[~nan], ref[~nan])
+
+
+@pytest.mark.parametrize("rows,D", [(2047, 2560), (2048, 2560), (2049, 2560), (2049, 2568)])
+def test_rmsnorm_two_rows_a_wave_up_to_2560(gpu, rows, D):
+    rng = np.random.default_rng(rows + D)
+    x, g = draw(rng, rows, D, std=2.0), (1 + 0.1 * rng.standard_normal(D)).astype(np.float32)
+    out, xd, gd = torch.zeros(rows * D + 8, dtype=torch.int16, device="cuda"), up(x), up(g)
+    lib().hip_rmsnorm(out.data_ptr(), xd.data_ptr(), gd.data_ptr(), rows, D, 1e-6)
+    got = down(out)
+    np.testing.assert_array_equal(got[:rows * D].reshape(rows, D), O.rmsnorm(x, g, 1e-6))
+    assert not got[rows * D:].any()
