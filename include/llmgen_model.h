@@ -14,8 +14,9 @@
  *   hip_sample       src/backend/cuda/sample/sample.zig:4-14          (CPU: src/backend/cpu/sample.zig:12-40)
  * Conventions are those of llmgen_attn.h: device pointers, bf16 as uint16_t bits, launches on the library
  * stream, no allocation and no synchronisation (capturable); unsupported shapes print one line to stderr and
- * launch nothing.  Every f32 operation is a separately rounded IEEE multiply, add, divide or square root (no
- * fused multiply-add), as in the reference's Zig code.
+ * launch nothing.  Every result is that of separately rounded IEEE f32 multiplies, adds, divides and square roots, as
+ * in the reference's Zig code (the products of hip_linear are fused multiply-adds only where the product is exact, which
+ * gives the same bits).
  */
 #ifndef LLMGEN_MODEL_H
 #define LLMGEN_MODEL_H

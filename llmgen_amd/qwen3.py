@@ -216,7 +216,8 @@ class Qwen3:
         ids_ptr = self.meta_dev.data_ptr() + lay.ids
         H, nq, nkv, hd, F = cfg.hidden, cfg.n_head, cfg.n_kv_head, cfg.head_dim, cfg.ffn
         x = self._empty(T, H)
-        xn, o = self._empty(T, H), self._empty(T, H)
+        xn = self._empty(T, H)
+        o = None if fused_qk else self._empty(T, H)
         q, k, v = self._empty(T, nq, hd), self._empty(T, nkv, hd), self._empty(T, nkv, hd)
         attn = self._empty(T, nq, hd)
         gate, up = self._empty(T, F), self._empty(T, F)
