@@ -379,8 +379,8 @@ template <class Op>
 void elementwise(bf16_t *out, const bf16_t *a, const bf16_t *b, size_t n, Op op) {
     if (n == 0) return;
     // Short streams are bound by the latency of one lane's work, and a value per lane is the least of it (SiLU of 16385 values
-    // 1.88 us, 1.97 in vectors; of 2^17 1.95 and 2.00, but add 1.97 and 1.83).
-    if (n <= 65536 || (((uintptr_t)out | (uintptr_t)a | (uintptr_t)b) & 15)) {
+    // 1.91 us, 1.97 in vectors, of 2^17 1.92 and 2.03, add 1.95 either way; of 2^20 2.77 and 2.61, add 2.69 and 2.17).
+    if (n <= 131072 || (((uintptr_t)out | (uintptr_t)a | (uintptr_t)b) & 15)) {
         elementwise_single_kernel<<<blocks_for(n, 256), 256, 0, g_llmgen_stream>>>(out, a, b, n, op);
         return;
     }

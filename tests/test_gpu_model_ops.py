@@ -221,8 +221,8 @@ def test_sample_slices_rule_edges(gpu, S, V):
     assert lib().hip_last_error() == 0
 
 
-# a value per lane up to 65536 values, vectors of eight beyond, where all three addresses allow them (offset 8 does)
-@pytest.mark.parametrize("n", [65535, 65536, 65537, 65544, 70007, 300001])
+# a value per lane up to 2^17 values, vectors of eight beyond, where all three addresses allow them (offset 8 does)
+@pytest.mark.parametrize("n", [65537, 131071, 131072, 131073, 131080, 140007, 300001])
 @pytest.mark.parametrize("offset", [0, 1, 8])
 def test_elementwise_long_streams(gpu, n, offset):
     rng = np.random.default_rng(n)
@@ -245,7 +245,7 @@ def silu(bits, up_bits=None):
         return s if up_bits is None else O.f32_to_bf16(O.bf16_to_f32(s) * O.bf16_to_f32(up_bits))
 
 
-@pytest.mark.parametrize("copies", [1, 2])  # a value per lane, vectors
+@pytest.mark.parametrize("copies", [1, 3])  # a value per lane, vectors
 def test_silu_and_silu_mul_every_gate(gpu, copies):
     """All 65536 gates, in both kernels of both ops, against the form with a double exp rounded once."""
     gates = np.tile(np.arange(65536, dtype=np.uint32).astype(np.uint16), copies)
