@@ -618,11 +618,12 @@ void linear_short_launch(LinArgs a) {
 
 // Tiles of the throughput-bound sizes.  A launch takes about as long as the CU with the most tiles:
 // ceil(tiles / CUs) * blocks of a tile / rate, where `rate` is the share of the matrix cores' peak that the tile
-// reached on sizes it fits (launch time taken off): 0.68 for 32 x 32 (631 x 1024 x 3072: 47.8 us; 350 x 1024 x 3072:
-// 34.4 us), 0.76 for 32 x 96 (2051 x 1024 x 1024: 43.2 us; 32 x 151936 x 1024: 102 us), 0.80 for 64 x 64 (997 x 1024 x
-// 3072: 56.5 us), 0.83 for 64 x 192 (997 x 3072 x 1024: 53.6 us) and 0.85 for 128 x 128 (2048 x 6144 x 2048: 385 us =
-// 134 TFLOP/s).  Larger tiles stage less per product but quantise coarser.  All five stage in whole slots per wave (a
-// slot that only some waves have splits the step's schedule: 96 x 32 with a 64-value chunk 10 % slower).
+// reached on sizes it fits (launch time taken off): 0.68 for 32 x 32 (350 x 1024 x 3072: 34 us), 0.76 for 32 x 96 (2051 x
+// 1024 x 1024: 43 to 48 us, by how warm the chip is), 0.80 for 64 x 64 (997 x 1024 x 3072: 57 to 66 us), 0.83 for 64 x 192
+// (997 x 3072 x 1024: 54 to 63 us) and 0.85 for 128 x 128 (2048 x 6144 x 2048: 371 to 385 us = 134 to 139 TFLOP/s).  Larger
+// tiles stage less per product but quantise coarser.  Of 92 sizes spread over M 17..3066, N 768..11480 and K 256..8192 the
+// chosen tile is 1.4 % slower than the best of the five on average, 7.8 % at most.  All five stage in whole slots per wave
+// (a slot that only some waves have splits the step's schedule: 96 x 32 with a 64-value chunk 10 % slower).
 struct LinChoice {
     int tm, tn;
     float rate;
